@@ -143,6 +143,11 @@ __device__ __forceinline__ int lane_id_here() {
   return l;
 }
 
+// v += s in place (volatile: not moved up, and no second register).
+__device__ __forceinline__ void add_here(uint32_t& v, uint32_t s) {
+  asm volatile("v_add_u32 %0, %1, %0" : "+v"(v) : "s"(s));
+}
+
 // A 16-byte-per-lane direct-to-LDS load written as inline asm, for the tile
 // scales: issued through the builtin, the compiler would treat every later
 // LDS read as possibly aliasing it and wait for vmcnt(0) first -- at the
@@ -243,12 +248,23 @@ __device__ __forceinline__ void tile_coords(int64_t pid, int64_t nt, int64_t til
 // would queue behind the next tile's ring loads: vmcnt retires in order)
 // and holds no scale registers through the K loop.  Returns whether a fast
 // path ran (and so issued exactly gemm_staged_stores<> stores per wave).
+//
+// RAGGED (launches whose last row tile is partial) lets that tile take the
+// same path: the stores' and residual loads' row steps ride in the per-lane
+// offset, which the buffer range check covers, and the range ends with row
+// M - 1, so rows past it are dropped.  The bounds-checked path such tiles took
+// before (2-byte stores, a scale load per output) set the pace of the whole
+// launch: the gate_up and down products of a 1001-row MLP (hidden 2048,
+// intermediate 6144) with its two row kernels 129.3 us, now 76.8.  A variant
+// of its own because the added offset arithmetic (one VALU add per 16-byte
+// store) makes the 256 x 256 SiLU kernel spill: 4096 rows 186 -> 192 us with
+// it.
 template <int OUT, int EPI, int FN, int FM>
 constexpr int gemm_staged_stores() {
   return OUT == FR_DTYPE_FP32 ? 4 * FN * FM : (EPI == kEpiSilu ? FN * FM : 2 * FN * FM);
 }
 
-template <int BN, int BM, int WN, int WM, int OUT, int EPI, int SRB>
+template <int BN, int BM, int WN, int WM, int OUT, int EPI, int SRB, bool RAGGED>
 __device__ __forceinline__ bool gemm_epilogue(const GemmArgs& g, v16f (&acc)[WN / 32][WM / 32], int64_t tm,
                                               int64_t tn, int wn, int wm, uint8_t* scl, uint8_t* stg,
                                               bool sa_vec, bool sb_vec, float sa0, float sb0) {
@@ -263,7 +279,7 @@ __device__ __forceinline__ bool gemm_epilogue(const GemmArgs& g, v16f (&acc)[WN 
   // registers to spare for it (not the 256 x 256 tile); others take the
   // bounds-checked path for it
   constexpr bool kResFast = !(BN == 256 && BM == 256);
-  const bool fast = tm * BM + BM <= g.M && tn * BN + BN <= g.N && g.bias == nullptr &&
+  const bool fast = (RAGGED || tm * BM + BM <= g.M) && tn * BN + BN <= g.N && g.bias == nullptr &&
                     (!RES || (kResFast && (g.ldr * EB) % 16 == 0 &&
                               (reinterpret_cast<uintptr_t>(g.res) & 15) == 0 && g.ldr < (int64_t(1) << 22))) &&
                     (g.ldo * EB) % 16 == 0 && (reinterpret_cast<uintptr_t>(g.out) & 15) == 0 &&
@@ -367,14 +383,24 @@ __device__ __forceinline__ bool gemm_epilogue(const GemmArgs& g, v16f (&acc)[WN 
   const uint32_t stg_base = lds_addr(stg);
   // stores through a buffer resource based at this wave's sub-tile: the
   // lane's offset is formed once, each store's row/column step is a scalar
-  // offset (no 64-bit address arithmetic per store)
+  // offset (no 64-bit address arithmetic per store).  RAGGED: the steps are
+  // added to the lane's offset in place, and the range ends with the last
+  // row's last column (an offset in a row past M is beyond it: N <= ldo)
+  auto range = [&](int64_t ld, int64_t ncols) __attribute__((always_inline)) -> uint32_t {
+    const int64_t mrows = g.M - m0;  // rows of this sub-tile and below
+    if (!RAGGED || mrows >= WM) return 0xFFFFFFFFu;
+    const int64_t end = mrows > 0 ? ((mrows - 1) * ld + ncols) * EB : 0;
+    return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(end));
+  };
   const uint64_t obase = reinterpret_cast<uint64_t>(static_cast<uint8_t*>(g.out) + (m0 * g.ldo + n0 / OD) * EB);
   const uint32_t olo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(obase));
   const uint32_t ohi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(obase >> 32));
   const __amdgpu_buffer_rsrc_t ro =
-      make_rsrc(reinterpret_cast<const void*>((static_cast<uint64_t>(ohi) << 32) | olo), 0xFFFFFFFFu);
+      make_rsrc(reinterpret_cast<const void*>((static_cast<uint64_t>(ohi) << 32) | olo),
+                range(g.ldo, (g.N - n0) / OD));
   const uint32_t ldo32 = static_cast<uint32_t>(g.ldo);
-  const uint32_t vo = ((lx / CPRSO) * ldo32 + (lx % CPRSO) * (16 / EB)) * EB;
+  uint32_t vo_at = 0;  // RAGGED: the step of the last store, contained in vo
+  uint32_t vo = ((lx / CPRSO) * ldo32 + (lx % CPRSO) * (16 / EB)) * EB;
   uint32_t ra[NRO];
 #pragma unroll
   for (int rr = 0; rr < NRO; ++rr) {
@@ -384,10 +410,10 @@ __device__ __forceinline__ bool gemm_epilogue(const GemmArgs& g, v16f (&acc)[WN 
   // scales: sa of the wave's rows up front, sb per column group
   u32x4 sb4[NQ];
   float sam_r[FM];
-  // fp16 outputs: the conversion's extra registers make the compiler spill
-  // in this epilogue, and a spilled register of a read still in flight would
-  // be stored stale, so that variant waits inside each read
-  constexpr bool kSafeReads = OUT == FR_DTYPE_FP16;
+  // fp16 outputs and the ragged 256 x 256 SiLU tile: the extra registers make
+  // the compiler spill in this epilogue, and a spilled register of a read
+  // still in flight would be stored stale, so these wait inside each read
+  constexpr bool kSafeReads = OUT == FR_DTYPE_FP16 || (RAGGED && SILU && BN == 256 && BM == 256);
   auto load_sb = [&](int cg) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < NQ; ++u) {
@@ -486,17 +512,18 @@ __device__ __forceinline__ bool gemm_epilogue(const GemmArgs& g, v16f (&acc)[WN 
   const uint32_t rlo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(rbase));
   const uint32_t rhi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(rbase >> 32));
   const __amdgpu_buffer_rsrc_t rres =
-      make_rsrc(reinterpret_cast<const void*>((static_cast<uint64_t>(rhi) << 32) | rlo), 0xFFFFFFFFu);
+      make_rsrc(reinterpret_cast<const void*>((static_cast<uint64_t>(rhi) << 32) | rlo), range(g.ldr, g.N - n0));
   const uint32_t ldr32 = static_cast<uint32_t>(g.ldr);
   const uint32_t vr = ((lx / CPRS) * ldr32 + (lx % CPRS) * (16 / EB)) * EB;
   u32x4 rv[2][NR];
   auto load_res = [&](int t) __attribute__((always_inline)) {
     const int cg = t / FM, j = t % FM;
 #pragma unroll
-    for (int rr = 0; rr < NR; ++rr)
+    for (int rr = 0; rr < NR; ++rr) {
+      const uint32_t to = ((j * 32 + rr * RPR) * ldr32 + cg * CPP) * EB;
       rv[t & 1][rr] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                     rres, vr, static_cast<int>(((j * 32 + rr * RPR) * ldr32 + cg * CPP) * EB), 0));
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rres, RAGGED ? vr + to : vr, RAGGED ? 0 : static_cast<int>(to), 0));
+    }
   };
   auto add_res = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
@@ -568,9 +595,14 @@ __device__ __forceinline__ bool gemm_epilogue(const GemmArgs& g, v16f (&acc)[WN 
     // not read back by this kernel; 2-3 % faster on the 4096-row gate_up,
     // down and M = 512 shapes, the decode step unchanged
 #pragma unroll
-    for (int rr = 0; rr < NRO; ++rr)
-      __builtin_amdgcn_raw_buffer_store_b128(w[rr], ro, vo,
-                                             static_cast<int>(((j * 32 + rr * RPRO) * ldo32 + cg * CPPO) * EB), kNT);
+    for (int rr = 0; rr < NRO; ++rr) {
+      const uint32_t to = ((j * 32 + rr * RPRO) * ldo32 + cg * CPPO) * EB;
+      if constexpr (RAGGED) {
+        if (t + rr > 0) add_here(vo, to - vo_at);
+        vo_at = to;
+      }
+      __builtin_amdgcn_raw_buffer_store_b128(w[rr], ro, vo, RAGGED ? 0 : static_cast<int>(to), kNT);
+    }
     if (t + 1 < NP) {
       stage();
       read_back();

@@ -39,9 +39,9 @@ namespace fr {
 // BN: weight rows (output columns) per tile, BM: activation rows per tile,
 // RB: bytes of K per LDS row (64: one MFMA K step per ring slot, 128: two,
 // so each direct-to-LDS load covers whole 128-byte lines), NSL: ring depth
-// in slots, KTAIL: K % 128 != 0 (the last K steps are partly or wholly
-// zero-filled).  EPI: kEpiPlain, kEpiRes or kEpiSilu.
-template <int BN, int BM, int NSL, int RB, int OUT, bool KTAIL, int EPI>
+// in slots, EDGE: K % 128 != 0 (the last K steps are partly or wholly
+// zero-filled) or M % BM != 0 (gemm_epilogue's RAGGED).  EPI: kEpiPlain, kEpiRes or kEpiSilu.
+template <int BN, int BM, int NSL, int RB, int OUT, bool EDGE, int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_fp8_mfma(GemmArgs g) {
   // The host pass only needs the kernel's signature (for its launch stub);
   // the body uses device-only buffer-resource builtins.
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_mfma(GemmArgs g) {
     uint8_t* sb = smem + slot * STAGE;
     uint8_t* sa = sb + BN * RB;
     const uint32_t k0 = static_cast<uint32_t>(lk) * RB;
-    const bool kin = !KTAIL || (k0 + lchunk * 16 < static_cast<uint64_t>(g.K));
+    const bool kin = !EDGE || (k0 + lchunk * 16 < static_cast<uint64_t>(g.K));
     if (l < IB) {
       const uint32_t o = lob[l] + (next ? bb_nxt : bb_cur);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(sb + (l * 4 + wave) * 1024), 16,
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_mfma(GemmArgs g) {
   auto epilogue = [&](int64_t local) -> bool __attribute__((always_inline)) {
     int64_t tm, tn;
     tile_coords(blockIdx.x + local * G, nt, tilesM, tm, tn);
-    return gemm_epilogue<BN, BM, WN, WM, OUT, EPI, SRB>(g, acc, tm, tn, wn, wm, scl + (local & 1) * 2048, stg,
+    return gemm_epilogue<BN, BM, WN, WM, OUT, EPI, SRB, EDGE>(g, acc, tm, tn, wn, wm, scl + (local & 1) * 2048, stg,
                                                          sa_vec, sb_vec, sa0, sb0);
   };
 
@@ -461,7 +461,7 @@ static hipError_t launch_mfma(const GemmArgs& g, hipStream_t st) {
   // with fewer K steps per tile than that, give every tile its own workgroup.
   const int64_t kt = ((g.K + 2 * kBK - 1) / (2 * kBK)) * 2;
   const unsigned grid = static_cast<unsigned>(nt < cus || kt < NSL * (RB / kBK) ? nt : cus);
-  if (g.K % (2 * kBK) == 0)
+  if (g.K % (2 * kBK) == 0 && g.M % BM == 0)
     hipLaunchKernelGGL((gemm_fp8_mfma<BN, BM, NSL, RB, OUT, false, EPI>), dim3(grid), dim3(256), 0, st, g);
   else
     hipLaunchKernelGGL((gemm_fp8_mfma<BN, BM, NSL, RB, OUT, true, EPI>), dim3(grid), dim3(256), 0, st, g);

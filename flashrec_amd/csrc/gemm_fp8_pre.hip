@@ -87,10 +87,11 @@ __device__ __forceinline__ void tile_coords_pre(int64_t pid, int64_t nt, int64_t
 }
 
 // BN: weight rows (output columns) per tile, BM: activation rows, NSL: ring
-// slots, KTAIL: K % 256 != 0 (activation chunks past K read as zero: the
-// prearranged K steps come in groups of 4), EPI: epilogue variant, WS: weight
+// slots, EDGE: K % 256 != 0 (activation chunks past K read as zero: the
+// prearranged K steps come in groups of 4) or M % BM != 0 (a partial last row
+// tile, gemm_epilogue's RAGGED), EPI: epilogue variant, WS: weight
 // register sets (step s loads step s + WS - 1's weights).
-template <int BN, int BM, int NSL, int OUT, bool KTAIL, int EPI, int WS>
+template <int BN, int BM, int NSL, int OUT, bool EDGE, int EPI, int WS>
 __global__ __launch_bounds__(256, 1) void gemm_fp8_pre(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int RB = 128;        // bytes of K per LDS row: two MFMA steps per slot
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_pre(GemmArgs g) {
   auto issue_a = [&](int slot, int lk, bool next, int i) __attribute__((always_inline)) {
     uint8_t* sa = smem + slot * STAGE;
     const uint32_t k0 = static_cast<uint32_t>(lk) * RB;
-    const bool kin = !KTAIL || (k0 + lchunk * 16 < static_cast<uint64_t>(g.K));
+    const bool kin = !EDGE || (k0 + lchunk * 16 < static_cast<uint64_t>(g.K));
     const uint32_t o = loa[i] + (next ? ba_nxt : ba_cur);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(sa + (i * 4 + wave) * 1024), 16, kin ? o : kOOB, k0,
                                              0, 0);
@@ -229,8 +230,8 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_pre(GemmArgs g) {
   auto epilogue = [&](int64_t local) __attribute__((always_inline)) {
     int64_t tm, tn;
     tile_coords_pre(blockIdx.x + local * G, nt, tilesM, multi_round, tm, tn);
-    gemm_epilogue<BN, BM, WN, WM, OUT, EPI, SRB>(g, acc, tm, tn, wn, wm, scl + (local & 1) * SCB, stg, sa_vec,
-                                                 sb_vec, sa0, sb0);
+    gemm_epilogue<BN, BM, WN, WM, OUT, EPI, SRB, EDGE>(g, acc, tm, tn, wn, wm, scl + (local & 1) * SCB, stg,
+                                                       sa_vec, sb_vec, sa0, sb0);
   };
 
   // ---- step schedule.  Step s (K step kt of its tile, ring slot s / 2,
@@ -389,7 +390,7 @@ static hipError_t launch_pre(const GemmArgs& g, hipStream_t st) {
   // four weight register sets (loads 3 steps ahead); eight on the smaller
   // tiles, whose steps are half as long, measured 2-5 % slower on the down
   // and o shapes
-  if (g.K % (64 * kPreSteps) == 0)
+  if (g.K % (64 * kPreSteps) == 0 && g.M % BM == 0)
     hipLaunchKernelGGL((gemm_fp8_pre<BN, BM, NSL, OUT, false, EPI, 4>), dim3(grid), dim3(256), 0, st, g);
   else
     hipLaunchKernelGGL((gemm_fp8_pre<BN, BM, NSL, OUT, true, EPI, 4>), dim3(grid), dim3(256), 0, st, g);
