@@ -36,6 +36,11 @@ struct GemmArgs {
   int silu;
 };
 
+// gemm_fp8_small.hip: runs the product where its rule on (M, N, K) takes it
+// (`taken`); operand conditions as the MFMA kernels'.  Both weight layouts
+// (`pre`: prearranged, else [N, K] rows) follow one rule and add in one order.
+hipError_t gemm_small(const GemmArgs& g, int out_dtype, bool pre, hipStream_t st, bool& taken);
+
 constexpr int kBK = 64;  // bytes of K per MFMA step
 // Epilogue variants (a compile-time kernel parameter, so the plain kernels
 // carry none of the others' code): the scaled product; the same plus a

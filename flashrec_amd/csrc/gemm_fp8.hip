@@ -482,6 +482,10 @@ static hipError_t dispatch(const GemmArgs& g, hipStream_t st) {
                        dim3(256), 0, st, g);
     return hipGetLastError();
   }
+  // few tiles: K split inside the workgroup (gemm_fp8_small.hip)
+  bool taken = false;
+  const hipError_t small = gemm_small(g, OUT, false, st, taken);
+  if (taken) return small;
   // Tile choice: the shape with the least estimated time, rounds of tiles
   // over the CUs (persistent workgroups: a partial round costs a full one)
   // times a tile's MFMA work over its relative efficiency (256x256 1.0,

@@ -403,7 +403,8 @@ static hipError_t launch_pre(const GemmArgs& g, hipStream_t st) {
 // (operands rotated through HBM): 256x256 1.0; 256x128 0.75 (the down and o
 // projections: 2218-2243 and 1553-1738 TFLOP/s against 1506-1605 and
 // 1225-1267 on 256x256 tiles, which leave half the CUs idle there); 128x128
-// 0.6 (slower than 256x128 on every shape measured; taken by small launches).
+// 0.6 (slower than 256x128 on every shape measured; taken by small launches
+// that the K-split tiles of gemm_fp8_small.hip do not take).
 template <int OUT, int EPI>
 static hipError_t dispatch_pre(const GemmArgs& g, hipStream_t st) {
   const int64_t cus = num_cus();
@@ -475,7 +476,11 @@ extern "C" int fr_fp8_scaled_mm_prearranged(const void* a, int64_t lda, const vo
   g.ldr = ldr;
   g.silu = silu ? 1 : 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipError_t err;
+  if (out_dtype != FR_DTYPE_BF16 && out_dtype != FR_DTYPE_FP16 && out_dtype != FR_DTYPE_FP32) return FR_EINVAL;
+  // few tiles: K split inside the workgroup (gemm_fp8_small.hip)
+  bool taken = false;
+  hipError_t err = gemm_small(g, out_dtype, true, st, taken);
+  if (taken) return err == hipSuccess ? FR_OK : FR_ELAUNCH;
   switch (out_dtype) {
     case FR_DTYPE_BF16:
       err = silu ? dispatch_pre<FR_DTYPE_BF16, kEpiSilu>(g, st)
