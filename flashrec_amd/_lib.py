@@ -104,6 +104,12 @@ SIGNATURES = {
         _P, _I64, _P, _I64, _I64, _I64, _I64, _F32, _P, _P,  # codes, ldq, scales, T, Hq, Hk, D, scale, plan, stream
     ],
     "fr_paged_attention_plan_size": [_I64, _I64, _I64],
+    "fr_paged_attention_waves": [_I64, _I64, _I64, _I64],
+    "fr_paged_attention_split_fp8": [
+        _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64,  # q, k_cache, v_cache + strides
+        _I64, _P, _P, _P,  # num_slots, kv_indices, kv_start, kv_len
+        _P, _I64, _I64, _I64, _I64, _I64, _I64, _F32, _P, _I32, _P,  # out + strides, T .. scale, plan, waves, stream
+    ],
     "fr_calib_mfma_ceiling": [_I64, _I64, _I32, _P, _P, _P],
     "fr_paged_attention_plan": [_P, _P, _P, _I64, _I64, _I64, _P, _P],
 }

@@ -17,7 +17,7 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
-from flashrec_amd._lib import Unsupported, call, load, require_device, stream_of
+from flashrec_amd._lib import DTYPE_CODE, Unsupported, call, load, require_device, stream_of
 
 
 class AttentionBackend:
@@ -242,7 +242,8 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     kernel: the o projection's e4m3 input ``[T, Hq * D]`` and its scales
     ``[T, 1]`` (qwen3.py:131-134 -> linear.py:118-151), bit-for-bit the two
     steps' result.  Head layouts the fused kernel does not take (more than 8
-    kv heads, 8 query heads per kv head) run the two steps."""
+    kv heads, 8 query heads per kv head), and launches with too few query
+    groups to fill the chip, run the two steps."""
     T, Hq, D, slots, Hk = _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len)
     if out is None:
         out = torch.empty(T, Hq * D, dtype=torch.float8_e4m3fn, device=q.device)
@@ -254,21 +255,27 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     if out_scale.dtype != torch.float32 or out_scale.numel() != T or not out_scale.is_contiguous():
         raise ValueError("out_scale must hold T contiguous fp32 values")
     require_device(out, out_scale)
-    try:
-        call("fr_paged_attention_quant_fp8",
-             q.data_ptr(), q.stride(0), q.stride(1),
-             k_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
-             v_cache.data_ptr(), v_cache.stride(0), v_cache.stride(1),
-             slots, kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
-             out.data_ptr(), out.stride(0), out_scale.data_ptr(),
-             T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk), stream_of(q))
-    except Unsupported:
-        from flashrec_amd.kernel.sglops import per_token_quant_fp8
-
-        o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, group_prefix=group_prefix)
-        codes, s = per_token_quant_fp8(o.reshape(T, Hq * D))
+    # where paged_attention splits its items' keys over waves, the quant runs
+    # on its rows (one more launch of 3 us; 512 rows over 1503 keys take 89 us
+    # fused and unsplit, 25 us so)
+    if int(load().fr_paged_attention_waves(T, Hq, Hk, kv_indices.numel())) == 1:
+        try:
+            call("fr_paged_attention_quant_fp8",
+                 q.data_ptr(), q.stride(0), q.stride(1),
+                 k_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
+                 v_cache.data_ptr(), v_cache.stride(0), v_cache.stride(1),
+                 slots, kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
+                 out.data_ptr(), out.stride(0), out_scale.data_ptr(),
+                 T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk), stream_of(q))
+            return out, out_scale
+        except Unsupported:
+            pass
+    o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, group_prefix=group_prefix)
+    codes = out if out.is_contiguous() else torch.empty((T, Hq * D), dtype=out.dtype, device=out.device)
+    call("fr_per_token_quant_fp8", o.data_ptr(), DTYPE_CODE[o.dtype], T, Hq * D, Hq * D, codes.data_ptr(),
+         out_scale.data_ptr(), stream_of(q))
+    if codes is not out:
         out.copy_(codes)
-        out_scale.copy_(s.reshape(out_scale.shape))
     return out, out_scale
 
 
@@ -286,11 +293,12 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     T, Hq, D, slots, Hk = _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len)
     if out is None:
         out = torch.empty(T, Hq, D, dtype=torch.bfloat16, device=q.device)
-    call("fr_paged_attention_fp8",
+    call("fr_paged_attention_split_fp8",
          q.data_ptr(), q.stride(0), q.stride(1),
          k_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
          v_cache.data_ptr(), v_cache.stride(0), v_cache.stride(1),
          slots, kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
          out.data_ptr(), out.stride(0), out.stride(1),
-         T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk), stream_of(q))
+         T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk),
+         int(load().fr_paged_attention_waves(T, Hq, Hk, kv_indices.numel())), stream_of(q))
     return out

@@ -11,16 +11,18 @@
 // sees P + j + 1.
 //
 // The work of one call goes in whole groups of 32 / NREP consecutive query
-// tokens (32 query rows):
-//  * paged_attn_grouped_d128 (bf16 MFMA) takes the groups whose tokens all
-//    see the same first 32 slots — beams of one request decoding over their
-//    shared prompt, the common case — and multiplies their shared slot
-//    prefix once for all 32 queries;
-//  * every other group is attended token by token on the VALU (attend_token):
-//    inside the same kernel for NREP < 8, by paged_attn_tokens_d128 (a
-//    second launch, more registers per wave) for NREP >= 8.
-// Arithmetic in fp32 (e4m3 and bf16 convert exactly; the MFMA path rounds the
-// probabilities to bf16, as the reference's bf16 SDPA does), output bf16.
+// tokens (32 query rows), each group and kv head an item of its own on bf16
+// MFMA (attend_segment).  The tokens of a group are taken in segments that
+// read common keys: one segment where all of them see the same first 32 slots
+// (beams of one request over their shared prompt, or a prompt's tokens at
+// 32 keys and more), else runs of tokens that share a slot list (the first
+// tokens of a prompt) or at least 32 leading slots (beams of two requests
+// meeting in a group), down to single tokens.  An item's key blocks are split
+// over NW waves of a workgroup when the items alone do not fill the chip.
+// Arithmetic in fp32 (e4m3 and bf16 convert exactly); the probabilities of
+// whole groups are rounded to bf16 (as the reference's bf16 SDPA does), those
+// of groups in several segments are carried as two bf16 terms (16 significant
+// bits).  Output bf16.
 #include <type_traits>
 
 #include "fr_common.h"
@@ -39,233 +41,38 @@ struct AttnArgs {
   uint16_t* out;            // [T, Hq, 128] bf16
   int64_t sot, soh;
   int64_t T, Hq, Hk, num_slots;
+  uint32_t row16;  // slot stride of both caches in 16-byte units, 0 where they differ or offsets pass 2^32
   float qscale;  // softmax scale * log2(e)
-  const int32_t* gp;  // [groups] shared prefix rounded down to 32 (0: none), or null
+  const int32_t* gp;  // [groups] slot prefix a group's tokens share, rounded down to 32, or null
 };
 
-// Sum over the 8 lanes of each aligned group of 8 (DPP: half-row mirror,
-// then quad swaps); every lane of the group gets the total.
-__device__ __forceinline__ float group8_sum(float v) {
-  v += __uint_as_float(static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), 0x141, 0xF, 0xF, false)));
-  v += __uint_as_float(static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), 0xB1, 0xF, 0xF, false)));
-  v += __uint_as_float(static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), 0x4E, 0xF, 0xF, false)));
-  return v;
-}
-
-// e4m3 x 16 (one 16-byte load) -> fp32, exact.
-__device__ __forceinline__ void e4m3x16_to_f32(const u32x4& w, float* f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[i]), false);
-    const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[i]), true);
-    f[4 * i + 0] = lo[0];
-    f[4 * i + 1] = lo[1];
-    f[4 * i + 2] = hi[0];
-    f[4 * i + 3] = hi[1];
-  }
-}
-
-// One (query token t, kv head kh) on the whole wave, VALU arithmetic, for
-// the NREP query heads that share kv head kh.  Lanes form 8 key groups of 8
-// lanes; a lane holds 16 of the 128 dims, so one key's K (or V) row for the
-// head is one 128-byte gather per group (16 bytes per lane).  Keys go in
-// chunks of 8 * NP: scores of a chunk stay in registers (pass 1, K), then the
-// chunk is folded into a running max / sum / accumulator (pass 2, V) in the
-// exp2 domain (q carries scale * log2(e)); the 8 key groups' partial sums
-// are merged once at the end.  Head kh * NREP + r's output row goes to
-// op0 + r * ohs (global memory, or the LDS staging of the quantizing kernel).
-template <int NREP, int NP>
-__device__ __forceinline__ void attend_token(const AttnArgs& a, int64_t t, int kh, int lane, uint16_t* op0,
-                                             int64_t ohs) {
-  const int kg = lane >> 3;       // key group
-  const int d0 = (lane & 7) * 16;  // first of this lane's 16 dims
-
-  // queries of the NREP heads sharing kv head kh, pre-scaled into the exp2 domain
-  float q[NREP][16];
-#pragma unroll
-  for (int r = 0; r < NREP; ++r) {
-    const uint16_t* qp = a.q + t * a.sqt + (kh * NREP + r) * a.sqh + d0;
-    const u32x4 w0 = *reinterpret_cast<const u32x4*>(qp);
-    const u32x4 w1 = *reinterpret_cast<const u32x4*>(qp + 8);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      q[r][2 * i] = __uint_as_float(w0[i] << 16) * a.qscale;
-      q[r][2 * i + 1] = __uint_as_float(w0[i] & 0xFFFF0000u) * a.qscale;
-      q[r][8 + 2 * i] = __uint_as_float(w1[i] << 16) * a.qscale;
-      q[r][8 + 2 * i + 1] = __uint_as_float(w1[i] & 0xFFFF0000u) * a.qscale;
-    }
-  }
-
-  const int32_t len = a.kv_len[t];
-  const int32_t* idx = a.kv_indices + a.kv_start[t];
-  float m[NREP], l[NREP], acc[NREP][16];
-#pragma unroll
-  for (int r = 0; r < NREP; ++r) {
-    m[r] = -__builtin_inff();
-    l[r] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[r][i] = 0.0f;
-  }
-
-  constexpr int CH = 8 * NP;  // keys per chunk
-  for (int c0 = 0; c0 < len; c0 += CH) {
-    // pass 1: scores of the chunk's keys (key c0 + 8p + kg in s[p])
-    int32_t slot[NP];
-    float s[NP][NREP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int key = c0 + 8 * p + kg;
-      int32_t sl = key < len ? idx[key] : -1;
-      if (sl >= a.num_slots) sl = -1;  // outside the pool: contributes nothing
-      slot[p] = sl;
-    }
-    u32x4 kw[NP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-      kw[p] = slot[p] >= 0 ? *reinterpret_cast<const u32x4*>(a.kc + static_cast<int64_t>(slot[p]) * a.skp + kh * a.skh + d0)
-                           : u32x4{0, 0, 0, 0};
-    float cm[NREP];
-#pragma unroll
-    for (int r = 0; r < NREP; ++r) cm[r] = -__builtin_inff();
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      float k[16];
-      e4m3x16_to_f32(kw[p], k);
-#pragma unroll
-      for (int r = 0; r < NREP; ++r) {
-        float d = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) d = __builtin_fmaf(q[r][i], k[i], d);
-        d = group8_sum(d);
-        s[p][r] = slot[p] >= 0 ? d : -__builtin_inff();
-        cm[r] = __builtin_fmaxf(cm[r], s[p][r]);
-      }
-    }
-    // chunk max over the 8 key groups (lanes 8 apart)
-#pragma unroll
-    for (int r = 0; r < NREP; ++r) {
-      cm[r] = __builtin_fmaxf(cm[r], __shfl_xor(cm[r], 8, 64));
-      cm[r] = __builtin_fmaxf(cm[r], __shfl_xor(cm[r], 16, 64));
-      cm[r] = __builtin_fmaxf(cm[r], __shfl_xor(cm[r], 32, 64));
-    }
-    // fold: rescale the running state to the new max
-    float mn[NREP];
-#pragma unroll
-    for (int r = 0; r < NREP; ++r) {
-      mn[r] = __builtin_fmaxf(m[r], cm[r]);
-      // mn is -inf only while every key so far is masked: keep the state zero
-      const float alpha = mn[r] == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f(m[r] - mn[r]);
-      l[r] *= alpha;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[r][i] *= alpha;
-      m[r] = mn[r];
-    }
-    // pass 2: probabilities and V
-    u32x4 vw[NP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-      vw[p] = slot[p] >= 0 ? *reinterpret_cast<const u32x4*>(a.vc + static_cast<int64_t>(slot[p]) * a.svp + kh * a.svh + d0)
-                           : u32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      float v[16];
-      e4m3x16_to_f32(vw[p], v);
-#pragma unroll
-      for (int r = 0; r < NREP; ++r) {
-        const float pr = slot[p] >= 0 ? __builtin_amdgcn_exp2f(s[p][r] - m[r]) : 0.0f;
-        l[r] += pr;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[r][i] = __builtin_fmaf(pr, v[i], acc[r][i]);
-      }
-    }
-  }
-
-  // merge the 8 key groups: sums over lanes 8, 16, 32 apart (each group's
-  // l counts its own keys once per lane of the group, identically)
-#pragma unroll
-  for (int r = 0; r < NREP; ++r) {
-    l[r] += __shfl_xor(l[r], 8, 64);
-    l[r] += __shfl_xor(l[r], 16, 64);
-    l[r] += __shfl_xor(l[r], 32, 64);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      acc[r][i] += __shfl_xor(acc[r][i], 8, 64);
-      acc[r][i] += __shfl_xor(acc[r][i], 16, 64);
-      acc[r][i] += __shfl_xor(acc[r][i], 32, 64);
-    }
-  }
-  if (kg != 0) return;
-#pragma unroll
-  for (int r = 0; r < NREP; ++r) {
-    // no visible key: zeros (the softmax of an empty row is undefined)
-    const float inv = l[r] > 0.0f ? 1.0f / l[r] : 0.0f;
-    u32x4 o0, o1;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      o0[i] = pack_bf16x2(acc[r][2 * i] * inv, acc[r][2 * i + 1] * inv);
-      o1[i] = pack_bf16x2(acc[r][8 + 2 * i] * inv, acc[r][8 + 2 * i + 1] * inv);
-    }
-    uint16_t* op = op0 + r * ohs + d0;
-    *reinterpret_cast<u32x4*>(op) = o0;
-    *reinterpret_cast<u32x4*>(op + 8) = o1;
-  }
-}
-
-// Whether every token of the group t0 .. t0 + ntok - 1 sees at least 32
-// slots and the same first 32 of them: the grouped kernel takes exactly
-// these groups (its shared prefix then has at least one 32-key block), the
-// per-token kernel all others.  Wave-uniform; both kernels call this.
+// Longest slot prefix shared by the `count` tokens from t0 on (count <= TOK).
+// Lanes 0 .. count-1 fetch the tokens' (start, length) in one load; every
+// comparison load of a 64-position chunk is issued before any is used.
 template <int TOK>
-__device__ __forceinline__ bool group_shares_block(const AttnArgs& a, int64_t t0, int lane) {
-  const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
+__device__ __forceinline__ int32_t tokens_prefix(const AttnArgs& a, int64_t t0, int count, int lane) {
   int32_t my_start = 0, my_len = 0x7FFFFFFF;
-  if (lane < ntok) {
+  if (lane < count) {
     my_start = a.kv_start[t0 + lane];
     my_len = a.kv_len[t0 + lane];
   }
   int32_t lenmin = my_len;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) lenmin = min(lenmin, __shfl_xor(lenmin, o, 64));
-  if (lenmin < 32) return false;
-  // lane p compares position p % 32 of tokens p / 32, p / 32 + 2, ...
-  const int pos = lane & 31;
-  const int32_t s0 = a.kv_indices[__builtin_amdgcn_readlane(my_start, 0) + pos];
-  bool ok = true;
-  for (int tt = 1 + (lane >> 5); tt < ntok; tt += 2)
-    ok = ok && a.kv_indices[__shfl(my_start, tt, 64) + pos] == s0;
-  return __ballot(!ok) == 0;
-}
-
-// Longest slot prefix shared by every token of the group starting at t0,
-// rounded down to a multiple of 32 (0 when the tokens do not share 32
-// slots).  Lanes 0 .. TOK-1 fetch the tokens' (start, length) in one load;
-// every comparison load of a 64-position chunk is issued before any is used.
-template <int TOK>
-__device__ __forceinline__ int32_t group_prefix32(const AttnArgs& a, int64_t t0, int lane) {
-  const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
-  int32_t my_start = 0, my_len = 0x7FFFFFFF;
-  if (lane < ntok) {
-    my_start = a.kv_start[t0 + lane];
-    my_len = a.kv_len[t0 + lane];
-  }
-  int32_t lenmin = my_len;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) lenmin = min(lenmin, __shfl_xor(lenmin, o, 64));
+  // unconditional loads (lists past the last token read the first token's,
+  // positions past the shortest list its last one): under a branch each would
+  // wait for the one before it
   int32_t starts[TOK];
 #pragma unroll
-  for (int tt = 0; tt < TOK; ++tt) starts[tt] = __builtin_amdgcn_readlane(my_start, tt);
-  const int32_t* i0 = a.kv_indices + starts[0];
+  for (int tt = 0; tt < TOK; ++tt) starts[tt] = __builtin_amdgcn_readlane(my_start, tt < count ? tt : 0);
   int32_t P = 0;
   for (int32_t c = 0; c < lenmin; c += 64) {
-    const int32_t pos = c + lane;
-    const bool in = pos < lenmin;
-    const int32_t s0 = in ? i0[pos] : 0;
+    const bool in = c + lane < lenmin;
+    const int32_t pos = in ? c + lane : lenmin - 1;
     int32_t sv[TOK];
 #pragma unroll
-    for (int tt = 1; tt < TOK; ++tt) sv[tt] = (in && tt < ntok) ? a.kv_indices[starts[tt] + pos] : s0;
+    for (int tt = 0; tt < TOK; ++tt) sv[tt] = a.kv_indices[starts[tt] + pos];
+    const int32_t s0 = sv[0];
     bool ok = in;
 #pragma unroll
     for (int tt = 1; tt < TOK; ++tt) ok = ok && sv[tt] == s0;
@@ -276,8 +83,44 @@ __device__ __forceinline__ int32_t group_prefix32(const AttnArgs& a, int64_t t0,
     }
     P = c + 64;
   }
-  P = min(P, lenmin);
-  return P & ~31;
+  return min(P, lenmin);
+}
+
+// The slot prefix shared by a whole group, rounded down to 32 (the plan's
+// entry).
+template <int TOK>
+__device__ __forceinline__ int32_t group_prefix32(const AttnArgs& a, int64_t t0, int lane) {
+  return tokens_prefix<TOK>(a, t0, static_cast<int>(min<int64_t>(TOK, a.T - t0)), lane) & ~31;
+}
+
+// Bit tt (1 .. count-1): token t0 + tt reads the slot list of token t0 + tt -
+// 1, or shares at least its first 32 slots.
+template <int TOK>
+__device__ __forceinline__ uint32_t linked_tokens(const AttnArgs& a, int64_t t0, int count, int lane) {
+  int32_t my_start = -1, my_len = 0;
+  if (lane < count) {
+    my_start = a.kv_start[t0 + lane];
+    my_len = a.kv_len[t0 + lane];
+  }
+  const int32_t prev = __shfl_up(my_start, 1, 64), plen = __shfl_up(my_len, 1, 64);
+  const bool in = lane > 0 && lane < count;
+  uint32_t linked = static_cast<uint32_t>(__ballot(in && my_start == prev));
+  const uint32_t tryit = static_cast<uint32_t>(__ballot(in && my_start != prev && my_len >= 32 && plen >= 32));
+  int32_t x[TOK], y[TOK];
+  const int pos = lane & 31;
+#pragma unroll
+  for (int tt = 1; tt < TOK; ++tt) {
+    // lists that are not to be looked at read a word that is there
+    const bool t = (tryit >> tt) & 1u;
+    const int32_t* const px = t ? a.kv_indices + __builtin_amdgcn_readlane(my_start, tt) + pos : a.kv_start + t0;
+    const int32_t* const py = t ? a.kv_indices + __builtin_amdgcn_readlane(my_start, tt - 1) + pos : a.kv_start + t0;
+    x[tt] = *px;
+    y[tt] = *py;
+  }
+#pragma unroll
+  for (int tt = 1; tt < TOK; ++tt)
+    if (((tryit >> tt) & 1u) && __ballot(x[tt] != y[tt]) == 0) linked |= 1u << tt;
+  return linked;
 }
 
 // The plan: one wave per group, the group's shared prefix for every layer.
@@ -291,28 +134,24 @@ __global__ __launch_bounds__(256) void attn_group_plan(AttnArgs a, int32_t* gp, 
 }
 
 // ---------------------------------------------------------------------------
-// Grouped kernel (the default): one wave per (group of 32 / NREP consecutive
-// query tokens, kv head), i.e. 32 query rows, on bf16 MFMA.
+// One wave per (group of 32 / NREP consecutive query tokens, kv head[, share
+// of the key blocks]), i.e. 32 query rows, on bf16 MFMA.
 //
-// Beams of one request share their prompt's slots, so consecutive decode
-// rows usually attend to a common slot prefix.  The wave finds the longest
-// prefix P shared by every token of its group (one ballot per 64 positions)
-// and runs it in blocks of 32 keys for all 32 queries at once:
-//   S^T[32 keys x 32 queries] = K . Q^T   (8 x mfma_f32_32x32x16_bf16; each
-//       lane gathers 64 bytes of one key row and converts them to bf16 with
-//       one op per two bytes; dims are taken in the order 64h + 8s + t on
-//       both operands, which leaves the dot products unchanged)
+// Blocks of 32 keys are multiplied for all 32 queries at once:
+//   K and V rows are gathered 8 whole rows per 16-byte load (8 lanes a row:
+//       a gather in fragment order touches 32 lines per load, and the address
+//       path, not the matrix work, then sets the block's time) and staged in
+//       wave-private LDS, the next block's gathers in flight meanwhile
+//   S^T[32 keys x 32 queries] = K . Q^T   (8 x mfma_f32_32x32x16_bf16; a lane
+//       reads 64 bytes of one key row and converts them to bf16 with one op
+//       per two bytes; dims are taken in the order 64h + 8s + t on both
+//       operands, which leaves the dot products unchanged)
 //   online softmax per query: a lane owns one query column and 16 key rows,
 //       so the block max takes one cross-lane step
-//   O^T[128 x 32] += V^T . P^T  (8 MFMAs; V is staged in LDS as bf16
-//       [key][dim] and read back transposed with ds_read_b64_tr_b16; the keys
-//       of each 16-key chunk are taken in the order the score layout holds
-//       them, so P^T feeds the B operand without a lane exchange)
-// The keys past the shared prefix run through the same block with each
-// token's own keys (NREP per token per block) and every query masked to its
-// own token's keys.  A shared 128-slot prefix is thus read and multiplied
-// once for all 32 queries (config-4 decode, 4096 beams: 25-29 us a layer,
-// against 189 us token by token).
+//   O^T[128 x 32] += V^T . P^T  (8 MFMAs; V is staged as bf16 [key][dim] and
+//       read back transposed with ds_read_b64_tr_b16; the keys of each 16-key
+//       chunk are taken in the order the score layout holds them, so P^T
+//       feeds the B operand without a lane exchange)
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -330,147 +169,163 @@ __device__ __forceinline__ bf16x8_t e4m3x8_to_bf16(uint32_t w0, uint32_t w1) {
                                             __builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, d)});
 }
 
-constexpr int kVRow = 288;  // LDS bytes per staged V row: 256 + 32 (bank spread)
+constexpr int kVRow = 288;   // LDS bytes per staged bf16 V row: 256 + 32 (bank spread)
+constexpr int kKRow = 144;   // LDS bytes per staged e4m3 K row: 128 + 16 (bank spread)
+constexpr int kStage = 32 * (kVRow + kKRow);  // one wave's staging
+
+// A run of consecutive tokens of a group that read common keys.
+struct Segment {
+  int32_t first, count;  // tokens of the group
+  int32_t shared;        // leading list positions that hold the same slots for all of them
+  bool one_list;         // the tokens read one slot list, each its own length of it
+};
+
+// What a lane knows about its query column n = lane % 32: token t0 + n / NREP,
+// head kh * NREP + n % NREP, and 64 of its 128 dims.
+struct Query {
+  u32x4 q[8];
+  int32_t start, len;  // the token's slot list (len 0 past the last token)
+  bool ok;
+};
 
 template <int NREP>
-constexpr bool kSeparateTokenKernel = NREP >= 8;
-
-// One (group, kv head kh) item on one wave; vs is the wave's 32 x kVRow
-// bytes of LDS.  STAGE: the 32 query rows' outputs go to vs (row n = query
-// column n, bf16 at byte 2 * dim) instead of a.out, for the quantizing
-// kernel below.
-template <int NREP, bool STAGE>
-__device__ __forceinline__ void grouped_item(const AttnArgs& a, uint8_t* vs, int64_t group, int kh, int lane) {
-  constexpr int TOK = 32 / NREP;  // tokens per group
-  const int64_t t0 = group * TOK;
-  const int n = lane & 31;  // query column (and key row when loading)
-  const int h = lane >> 5;  // half: dims 64h .. 64h + 63
-  // this lane's query and key token: t0 + n / NREP (head kh * NREP + n % NREP).
-  // Its row bounds and query are fetched before the plan entry is examined,
-  // so those loads share one latency with it.
-  const int64_t tq = t0 + n / NREP;
-  const bool qok = tq < a.T;
-  const int32_t qlen = qok ? a.kv_len[tq] : 0;
-  const int32_t* ik = a.kv_indices + (qok ? a.kv_start[tq] : 0);
-  const int32_t* i0 = a.kv_indices + a.kv_start[t0];
-  u32x4 qb[8];
-  {
-    const uint16_t* qp = a.q + (qok ? tq : 0) * a.sqt + (kh * NREP + n % NREP) * a.sqh + 64 * h;
+__device__ __forceinline__ Query load_query(const AttnArgs& a, int64_t t0, int kh, int lane) {
+  Query Q;
+  const int n = lane & 31, h = lane >> 5;
+  const int64_t t = t0 + n / NREP;
+  Q.ok = t < a.T;
+  Q.len = Q.ok ? a.kv_len[t] : 0;
+  Q.start = a.kv_start[Q.ok ? t : t0];
+  const uint16_t* qp = a.q + (Q.ok ? t : t0) * a.sqt + (kh * NREP + n % NREP) * a.sqh + 64 * h;
 #pragma unroll
-    for (int s = 0; s < 8; ++s)
-      qb[s] = qok ? *reinterpret_cast<const u32x4*>(qp + 8 * s) : u32x4{0, 0, 0, 0};
-  }
-  // A group without a shared 32-slot block is attended token by token on
-  // the VALU: here, by this wave for its kv head, when the per-token
-  // registers fit two waves per SIMD (NREP < 8); otherwise by
-  // paged_attn_tokens_d128, a launch of its own.
-  if (a.gp ? a.gp[group] == 0 : !group_shares_block<TOK>(a, t0, lane)) {
-    if constexpr (!kSeparateTokenKernel<NREP>) {
-      const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
-      for (int tt = 0; tt < ntok; ++tt) {
-        if constexpr (STAGE)
-          attend_token<NREP, 16 / NREP>(a, t0 + tt, kh, lane, reinterpret_cast<uint16_t*>(vs + tt * NREP * kVRow),
-                                        kVRow / 2);
-        else
-          attend_token<NREP, 16 / NREP>(a, t0 + tt, kh, lane, a.out + (t0 + tt) * a.sot + kh * NREP * a.soh,
-                                        a.soh);
-      }
-    }
-    return;
-  }
+  for (int s = 0; s < 8; ++s) Q.q[s] = Q.ok ? *reinterpret_cast<const u32x4*>(qp + 8 * s) : u32x4{0, 0, 0, 0};
+  return Q;
+}
 
-  // ---- shared slot prefix of the group's tokens: from the plan, or found here
-  const int32_t P32 = a.gp ? a.gp[group] : group_prefix32<TOK>(a, t0, lane);
-
-  // ---- running softmax state of this lane's query (the two halves hold the
-  // same m; l and O are per half: O^T rows 32mt + 8(v/4) + 4h + v%4)
-  float m = -__builtin_inff(), l = 0.0f;
+// Softmax state of a lane's query over the keys seen so far: both halves hold
+// the same m; l and O are per half (O^T rows 32 mt + 8 (v / 4) + 4 h + v % 4).
+struct Softmax {
+  float m, l;
   f32x16_t O[4];
+};
+
+// Block range [part * blocks / parts, (part + 1) * blocks / parts) of a
+// segment, for the queries of its tokens (the other columns' results mean
+// nothing).  FINE: probabilities as two bf16 terms, and `nan` reports a NaN
+// code in a V row that some of the segment's queries must not see (its product
+// with their zero probability would still be NaN).  `stage`: kStage bytes of
+// this wave's LDS.
+template <int NREP, bool FINE>
+__device__ __forceinline__ void attend_segment(const AttnArgs& a, uint8_t* stage, int kh, int lane, const Query& Q,
+                                               const Segment& seg, int part, int parts, Softmax& X, bool& nan) {
+  uint8_t* const vs = stage;
+  uint8_t* const ks = stage + 32 * kVRow;
+  const int n = lane & 31;  // query column, and key row when reading K
+  const int h = lane >> 5;  // half: dims 64h .. 64h + 63
+  const int tok = n / NREP;
+  const bool inseg = tok >= seg.first && tok < seg.first + seg.count;
+  const int32_t qlen = inseg ? Q.len : 0;
+  X.m = -__builtin_inff();
+  X.l = 0.0f;
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) O[mt][v] = 0.0f;
+    for (int v = 0; v < 16; ++v) X.O[mt][v] = 0.0f;
 
-  // Blocks of 32 key rows.  Block b < nshared: row n is the shared slot
-  // i0[32b + n] for every query; after that, row r holds position
-  // P32 + j * NREP + r % NREP (j = b - nshared) of token t0 + r / NREP and
-  // each query only sees its own token's rows.
-  const int32_t klen = qlen;
-  int32_t rest = klen - P32;
+  int32_t maxlen = qlen, minlen = inseg && Q.ok ? Q.len : 0x7FFFFFFF;
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) rest = max(rest, __shfl_xor(rest, o, 64));
-  const int32_t nshared = P32 / 32;
+  for (int o = 32; o >= 1; o >>= 1) {
+    maxlen = max(maxlen, __shfl_xor(maxlen, o, 64));
+    minlen = min(minlen, __shfl_xor(minlen, o, 64));
+  }
+  // Blocks of 32 key rows.  Block b < nshared: row r is position 32 b + r of
+  // the common list; after that, row r holds position shared + (b - nshared) *
+  // NREP + r % NREP of token r / NREP's own list, and each query only sees its
+  // own token's rows.
+  const int32_t P = seg.one_list ? maxlen : seg.shared;
+  const int32_t rest = seg.one_list ? 0 : maxlen - P;
+  const int32_t nshared = (P + 31) / 32;
   const int32_t nblocks = nshared + (rest > 0 ? (rest + NREP - 1) / NREP : 0);
+  const int32_t b0 = part * nblocks / parts, b1 = (part + 1) * nblocks / parts;
+  // blocks from here on hold rows that some query of the segment must not see
+  const int32_t clean = min(nshared, seg.one_list ? minlen / 32 : nshared);
+  const int32_t* const i0 = a.kv_indices + __builtin_amdgcn_readlane(Q.start, seg.first * NREP);
+  const int32_t* const ik = a.kv_indices + Q.start;
 
-  struct Loaded {
-    u32x4 kw[4], vw[4];
-    bool ok;
+  // Slot of key row n of block b (-1: none), fetched a block ahead of its
+  // gathers.  Gathers are unconditional (an invalid row reads slot 0's
+  // bytes); scores of invalid rows are masked and their V rows zeroed, so
+  // nothing from them (not even a NaN pattern) reaches the sums.
+  auto slot_of = [&](int32_t b) __attribute__((always_inline)) -> int32_t {
+    if (b >= b1) return -1;
+    if (b < nshared) {
+      const int32_t pos = 32 * b + n;
+      return pos < P ? i0[pos] : -1;
+    }
+    const int32_t pos = P + (b - nshared) * NREP + n % NREP;
+    return pos < qlen ? ik[pos] : -1;
   };
-  // Gathers are unconditional (an invalid row reads slot 0's bytes); scores
-  // of invalid rows are masked below and their V rows zeroed, so nothing
-  // from them (not even a NaN pattern) reaches the sums.
-  // Slot of this lane's key row in block bi (-1: none).  Fetched one block
-  // ahead, so its load latency overlaps the previous block's work (holding
-  // the next block's row gathers in registers as well measured no faster).
-  auto slot_of = [&](int32_t bi) __attribute__((always_inline)) -> int32_t {
-    if (bi < nshared) return i0[32 * bi + n];
-    const int32_t pos = P32 + (bi - nshared) * NREP + n % NREP;
-    return (bi < nblocks && pos < klen) ? ik[pos] : -1;
-  };
-  auto load = [&](int32_t slot, Loaded& L) __attribute__((always_inline)) {
-    L.ok = slot >= 0 && slot < a.num_slots;
-    const int64_t sl = L.ok ? slot : 0;
-    const uint8_t* kp = a.kc + sl * a.skp + kh * a.skh + 64 * h;
-    const uint8_t* vp = a.vc + sl * a.svp + kh * a.svh + 64 * h;
+  const int gr = lane >> 3;         // gathers: row 8 i + gr, bytes 16 (lane % 8) ..
+  const int gc = (lane & 7) * 16;
+  const uint8_t* const kbase = a.kc + kh * a.skh + gc;
+  const uint8_t* const vbase = a.vc + kh * a.svh + gc;
+  u32x4 kw[4], vw[4];
+  uint32_t rows_ok = 0;  // bit r: key row r of the gathered block usable
+  auto gather = [&](int32_t slot) __attribute__((always_inline)) {
+    const bool ok = slot >= 0 && slot < a.num_slots;
+    rows_ok = static_cast<uint32_t>(__ballot(ok));
+    const int32_t sl = ok ? slot : 0;
+    if (a.row16 != 0) {
+      // one pool layout, offsets in 16-byte units below 2^32: one multiply per
+      // block, made by the lane that holds the slot (quarter-rate: 64-bit
+      // products per gathered row took a third of the block's issue time)
+      const uint32_t off = static_cast<uint32_t>(sl) * a.row16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint64_t o = static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(off), 8 * i + gr, 64))) << 4;
+        kw[i] = *reinterpret_cast<const u32x4*>(kbase + o);
+        vw[i] = *reinterpret_cast<const u32x4*>(vbase + o);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      L.kw[i] = *reinterpret_cast<const u32x4*>(kp + 16 * i);
-      L.vw[i] = *reinterpret_cast<const u32x4*>(vp + 16 * i);
+      const int64_t s = __shfl(sl, 8 * i + gr, 64);
+      kw[i] = *reinterpret_cast<const u32x4*>(kbase + s * a.skp);
+      vw[i] = *reinterpret_cast<const u32x4*>(vbase + s * a.svp);
     }
   };
 
-  auto compute = [&](int32_t bi, Loaded& L, auto own_c) __attribute__((always_inline)) {
-    constexpr bool OWN = decltype(own_c)::value;
-    const int32_t pos_base = P32 + (bi - nshared) * NREP;
-    // bit r: key row r usable (lanes 32-63 load the same rows as 0-31)
-    const uint32_t rows_ok = static_cast<uint32_t>(__ballot(L.ok));
-    const bool all_rows = rows_ok == 0xFFFFFFFFu;
-    if (!all_rows) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) L.vw[i][w] = L.ok ? L.vw[i][w] : 0u;
-    }
+  // kind 0: every query sees every valid row; 1: rows below its own length;
+  // 2: its own token's rows
+  auto compute = [&](int32_t b, uint32_t ok_rows, auto kind_c) __attribute__((always_inline)) {
+    constexpr int KIND = decltype(kind_c)::value;
     // S^T = K . Q^T
     f32x16_t S;
 #pragma unroll
     for (int v = 0; v < 16; ++v) S[v] = 0.0f;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const bf16x8_t ka = e4m3x8_to_bf16(L.kw[s / 2][(s % 2) * 2], L.kw[s / 2][(s % 2) * 2 + 1]);
-      S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, __builtin_bit_cast(bf16x8_t, qb[s]), S, 0, 0, 0);
-    }
-    // V rows -> LDS as bf16 [key][dim]
-#pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bf16x8_t lo = e4m3x8_to_bf16(L.vw[i][0], L.vw[i][1]);
-      const bf16x8_t hi = e4m3x8_to_bf16(L.vw[i][2], L.vw[i][3]);
-      *reinterpret_cast<bf16x8_t*>(vs + n * kVRow + 128 * h + 32 * i) = lo;
-      *reinterpret_cast<bf16x8_t*>(vs + n * kVRow + 128 * h + 32 * i + 16) = hi;
+      const u32x4 w = *reinterpret_cast<const u32x4*>(ks + n * kKRow + 64 * h + 16 * i);
+      S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(w[0], w[1]),
+                                                  __builtin_bit_cast(bf16x8_t, Q.q[2 * i]), S, 0, 0, 0);
+      S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(w[2], w[3]),
+                                                  __builtin_bit_cast(bf16x8_t, Q.q[2 * i + 1]), S, 0, 0, 0);
     }
     // scores of this lane's query against key rows r = 8(v/4) + 4h + v%4,
     // unscaled (the scale is positive: the block max scales with them, and
     // each probability takes the scale in one fma)
     float x[16];
-    if (!OWN && all_rows) {
+    if (KIND == 0 && ok_rows == 0xFFFFFFFFu) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) x[v] = S[v];
     } else {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int r = 8 * (v / 4) + 4 * h + (v % 4);
-        bool ok = (rows_ok >> r) & 1u;
-        if (OWN) ok = ok && (r / NREP == n / NREP) && (pos_base + r % NREP < qlen);
+        bool ok = (ok_rows >> r) & 1u;
+        if (KIND == 1) ok = ok && 32 * b + r < qlen;
+        if (KIND == 2) ok = ok && r / NREP == tok && P + (b - nshared) * NREP + r % NREP < qlen;
         x[v] = ok ? S[v] : -__builtin_inff();
       }
     }
@@ -481,33 +336,39 @@ __device__ __forceinline__ void grouped_item(const AttnArgs& a, uint8_t* vs, int
     // Lazy rescale: probabilities are taken against the reference max m and
     // may reach 2^8; the accumulators are rescaled only when some query's
     // block max passes m + 8 (wave-uniform, so O is touched rarely).
-    const bool grow = mb > m + 8.0f;
+    const bool grow = mb > X.m + 8.0f;
     if (__ballot(grow)) {
-      const float mn = grow ? mb : m;
-      const float alpha = (m == -__builtin_inff()) ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
-      m = mn;
-      l *= alpha;
+      const float mn = grow ? mb : X.m;
+      const float alpha = (X.m == -__builtin_inff()) ? 0.0f : __builtin_amdgcn_exp2f(X.m - mn);
+      X.m = mn;
+      X.l *= alpha;
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) O[mt][v] *= alpha;
+        for (int v = 0; v < 16; ++v) X.O[mt][v] *= alpha;
     }
     // m stays -inf only while every row this query saw was masked; then
     // every x is -inf and the probabilities must be 0, not exp2(NaN)
-    const float mref = m == -__builtin_inff() ? 0.0f : m;
+    const float mref = X.m == -__builtin_inff() ? 0.0f : X.m;
     float pr[16];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       pr[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[v], a.qscale, -mref));  // x = -inf gives 0
-      l += pr[v];
+      X.l += pr[v];
     }
-    bf16x8_t pb[2];
+    bf16x8_t pb[2], pl[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      u32x4 w;
+      u32x4 w, lo;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) w[t] = pack_bf16x2(pr[8 * c + 2 * t], pr[8 * c + 2 * t + 1]);
+      for (int t = 0; t < 4; ++t) {
+        w[t] = pack_bf16x2(pr[8 * c + 2 * t], pr[8 * c + 2 * t + 1]);
+        if constexpr (FINE)
+          lo[t] = pack_bf16x2(pr[8 * c + 2 * t] - __uint_as_float(w[t] << 16),
+                              pr[8 * c + 2 * t + 1] - __uint_as_float(w[t] & 0xFFFF0000u));
+      }
       pb[c] = __builtin_bit_cast(bf16x8_t, w);
+      if constexpr (FINE) pl[c] = __builtin_bit_cast(bf16x8_t, lo);
     }
     // O^T += V^T . P^T; A[dim][k] through the transposing LDS read
     const int g = lane >> 4, i16 = lane & 15;
@@ -522,56 +383,277 @@ __device__ __forceinline__ void grouped_item(const AttnArgs& a, uint8_t* vs, int
             __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(vs + (r0 + 8) * kVRow + 2 * col));
         const bf16x8_t av = __builtin_bit_cast(
             bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        O[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pb[c], O[mt], 0, 0, 0);
+        X.O[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pb[c], X.O[mt], 0, 0, 0);
+        if constexpr (FINE) X.O[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pl[c], X.O[mt], 0, 0, 0);
       }
     }
   };
 
-  // One block's gathers at a time: holding a second block's gathers in
-  // registers (as a prefetch) needs 329 registers and one wave per SIMD;
-  // without it the kernel fits two waves per SIMD (launch bound below), and
-  // the other wave hides the gather latency (config-4 decode 62 -> 44 us).
-  Loaded LA;
-  int32_t bi = 0;
-  int32_t slot = nblocks > 0 ? slot_of(0) : -1;
-  for (; bi < nshared; ++bi) {
-    load(slot, LA);
-    if (bi + 1 < nblocks) slot = slot_of(bi + 1);
-    compute(bi, LA, std::false_type{});
+  if (b0 >= b1) return;
+  // the next block's gathers are in flight while a block is multiplied; the
+  // two-term form has no registers to spare for them
+  constexpr bool AHEAD = !FINE;
+  int32_t slot = slot_of(b0);
+  if (AHEAD) {
+    gather(slot);
+    slot = slot_of(b0 + 1);
   }
-  for (; bi < nblocks; ++bi) {
-    load(slot, LA);
-    if (bi + 1 < nblocks) slot = slot_of(bi + 1);
-    compute(bi, LA, std::true_type{});
-  }
-
-  // ---- normalise and store this lane's query (64 of its 128 dims)
-  const float lt = l + __shfl_xor(l, 32, 64);
-  if (!qok) return;
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-  uint16_t* op = STAGE ? reinterpret_cast<uint16_t*>(vs + n * kVRow)
-                       : a.out + tq * a.sot + (kh * NREP + n % NREP) * a.soh;
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x2 w;
-      w[0] = pack_bf16x2(O[mt][4 * j] * inv, O[mt][4 * j + 1] * inv);
-      w[1] = pack_bf16x2(O[mt][4 * j + 2] * inv, O[mt][4 * j + 3] * inv);
-      *reinterpret_cast<u32x2*>(op + 32 * mt + 8 * j + 4 * h) = w;
+  for (int32_t b = b0; b < b1; ++b) {
+    if (!AHEAD) {
+      gather(slot);
+      slot = slot_of(b + 1);
     }
+    const uint32_t ok_rows = rows_ok;
+    if (ok_rows != 0xFFFFFFFFu) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) vw[i][w] = (ok_rows >> (8 * i + gr)) & 1u ? vw[i][w] : 0u;
+    }
+    if (FINE && b >= clean) {
+      uint32_t bad = 0;  // some byte of magnitude 0x7F
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) bad |= ((vw[i][w] & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;
+      nan = nan || __ballot(bad != 0) != 0;
+    }
+    // rows -> LDS: K as it is, V as bf16 [key][dim]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 8 * i + gr;
+      *reinterpret_cast<u32x4*>(ks + r * kKRow + gc) = kw[i];
+      *reinterpret_cast<bf16x8_t*>(vs + r * kVRow + 2 * gc) = e4m3x8_to_bf16(vw[i][0], vw[i][1]);
+      *reinterpret_cast<bf16x8_t*>(vs + r * kVRow + 2 * gc + 16) = e4m3x8_to_bf16(vw[i][2], vw[i][3]);
+    }
+    if (AHEAD && b + 1 < b1) {
+      gather(slot);
+      slot = slot_of(b + 2);
+    }
+    if (b < clean) compute(b, ok_rows, std::integral_constant<int, 0>{});
+    else if (b < nshared) compute(b, ok_rows, std::integral_constant<int, 1>{});
+    else compute(b, ok_rows, std::integral_constant<int, 2>{});
+  }
 }
 
+// The segments of a group whose tokens do not all share 32 slots, in token
+// order: next() gives the one that starts at token `at`.
 template <int NREP>
-__global__ __launch_bounds__(256, 2) void paged_attn_grouped_d128(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * 32 * kVRow];
+struct Segments {
+  static constexpr int TOK = 32 / NREP;
+  const AttnArgs& a;
+  int64_t t0;
+  int lane, ntok;
+  uint32_t linked;
+  __device__ __forceinline__ Segments(const AttnArgs& a_, int64_t t0_, int lane_)
+      : a(a_), t0(t0_), lane(lane_), ntok(static_cast<int>(min<int64_t>(TOK, a_.T - t0_))) {
+    linked = linked_tokens<TOK>(a, t0, ntok, lane);
+  }
+  __device__ __forceinline__ Segment next(int at, const Query& Q, bool single) const {
+    Segment s{at, 1, 0, true};
+    if (single) return s;
+    while (at + s.count < ntok && ((linked >> (at + s.count)) & 1u)) ++s.count;
+    // one list for all of them?
+    const int32_t st = __builtin_amdgcn_readlane(Q.start, at * NREP);
+    const int tok = (lane & 31) / NREP;
+    const bool other = tok >= at && tok < at + s.count && Q.start != st;
+    if (__ballot(other) == 0) return s;
+    s.one_list = false;
+    s.shared = tokens_prefix<TOK>(a, t0 + at, s.count, lane);
+    return s;
+  }
+};
+
+// The whole group as one segment, from its shared prefix rounded down to 32:
+// the up to 31 shared positions past that join the common blocks (as own rows
+// they would take NREP keys a block: at 28 of them 14 blocks instead of one).
+template <int NREP>
+__device__ __forceinline__ Segment whole_group(const AttnArgs& a, int32_t p32, const Query& Q, int lane) {
+  constexpr int TOK = 32 / NREP;
+  const int32_t st = __builtin_amdgcn_readfirstlane(Q.start);
+  if (__ballot(Q.ok && Q.start != st) == 0) return Segment{0, TOK, p32, true};
+  int32_t minlen = Q.ok ? Q.len : 0x7FFFFFFF, maxlen = Q.len;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    minlen = min(minlen, __shfl_xor(minlen, o, 64));
+    maxlen = max(maxlen, __shfl_xor(maxlen, o, 64));
+  }
+  // at most two own blocks in any case: the look costs as much as they do
+  if (maxlen - p32 <= 2 * NREP) return Segment{0, TOK, p32, false};
+  // (every list holds p32 positions and more; a token past the last one
+  // repeats the first: Q.start)
+  const bool in = p32 + (lane & 31) < minlen;
+  const int32_t pos = in ? p32 + (lane & 31) : 0;
+  int32_t sv[TOK];
+#pragma unroll
+  for (int tt = 0; tt < TOK; ++tt) sv[tt] = a.kv_indices[__builtin_amdgcn_readlane(Q.start, tt * NREP) + pos];
+  bool ok = in;
+#pragma unroll
+  for (int tt = 1; tt < TOK; ++tt) ok = ok && sv[tt] == sv[0];
+  const uint32_t bad = static_cast<uint32_t>(__ballot(!ok));  // the two halves agree
+  return Segment{0, TOK, p32 + (bad ? __builtin_ctz(bad) : 32), false};
+}
+
+// A lane's normalised output row piece: 4 consecutive dims 32 mt + 8 j + 4 h ..
+// as bf16 (no visible key: zeros, the softmax of an empty row is undefined).
+__device__ __forceinline__ u32x2 out4(const Softmax& X, float inv, int mt, int j) {
+  return u32x2{pack_bf16x2(X.O[mt][4 * j] * inv, X.O[mt][4 * j + 1] * inv),
+               pack_bf16x2(X.O[mt][4 * j + 2] * inv, X.O[mt][4 * j + 3] * inv)};
+}
+
+// One item on one wave: the lane's query's 64 dims as 32 packed bf16 pairs.
+template <int NREP>
+__device__ __forceinline__ void attend_item(const AttnArgs& a, uint8_t* stage, int64_t group, int kh, int lane,
+                                            u32x2 (&o)[16]) {
+  const int64_t t0 = group * (32 / NREP);
+  const Query Q = load_query<NREP>(a, t0, kh, lane);
+  const int32_t gp = a.gp ? a.gp[group] : group_prefix32<32 / NREP>(a, t0, lane);
+  Softmax X;
+  bool nan = false;
+  if (gp > 0) {
+    attend_segment<NREP, false>(a, stage, kh, lane, Q, whole_group<NREP>(a, gp, Q, lane), 0, 1, X, nan);
+    const float lt = X.l + __shfl_xor(X.l, 32, 64);
+    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[i] = out4(X, inv, i >> 2, i & 3);
+    return;
+  }
+  const Segments<NREP> segs(a, t0, lane);
+  const int tok = (lane & 31) / NREP;
+  int single_until = 0;
+  for (int at = 0; at < segs.ntok;) {
+    const Segment s = segs.next(at, Q, at < single_until);
+    nan = false;
+    attend_segment<NREP, true>(a, stage, kh, lane, Q, s, 0, 1, X, nan);
+    if (nan && s.count > 1) {
+      single_until = at + s.count;
+      continue;
+    }
+    const float lt = X.l + __shfl_xor(X.l, 32, 64);
+    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+    if (tok >= at && tok < at + s.count) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[i] = out4(X, inv, i >> 2, i & 3);
+    }
+    at += s.count;
+  }
+}
+
+// Items on one wave each (launches with enough of them to fill the chip).
+template <int NREP>
+__global__ __launch_bounds__(64, 2) void paged_attn_d128(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kStage];
+  const int lane = threadIdx.x;
+  // last groups first: a causal prompt's longest items lead, the short ones
+  // fill the tail
+  const int64_t groups = (a.T + 32 / NREP - 1) / (32 / NREP);
+  const int64_t group = groups - 1 - blockIdx.x / a.Hk;
+  const int kh = static_cast<int>(blockIdx.x % a.Hk);
+  u32x2 o[16];
+  attend_item<NREP>(a, lds, group, kh, lane, o);
+  const int n = lane & 31, h = lane >> 5;
+  const int64_t t = group * (32 / NREP) + n / NREP;
+  if (t >= a.T) return;
+  uint16_t* const op = a.out + t * a.sot + (kh * NREP + n % NREP) * a.soh;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) *reinterpret_cast<u32x2*>(op + 8 * i + 4 * h) = o[i];
+}
+
+// An item's key blocks split over NW waves: each wave's softmax state over its
+// share, then the states merged through LDS (rescaled to the common max, added
+// in wave order) and the rows written by all threads.
+template <int NREP, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void paged_attn_split_d128(AttnArgs a) {
+  constexpr int kMerge = NW * 16384;  // 32 queries x 128 dims fp32 per wave
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kMerge > NW * kStage ? kMerge : NW * kStage];
+  __shared__ float ms[NW][32], ls[NW][32];
+  __shared__ int saw_nan;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + wave;
-  const int64_t group = item / a.Hk;
-  const int kh = static_cast<int>(item - group * a.Hk);
-  if (group * (32 / NREP) >= a.T) return;
-  grouped_item<NREP, false>(a, lds + wave * (32 * kVRow), group, kh, lane);
+  const int64_t groups = (a.T + 32 / NREP - 1) / (32 / NREP);
+  const int64_t group = groups - 1 - blockIdx.x / a.Hk;
+  const int kh = static_cast<int>(blockIdx.x % a.Hk);
+  const int64_t t0 = group * (32 / NREP);
+  const int n = lane & 31, h = lane >> 5;
+  const Query Q = load_query<NREP>(a, t0, kh, lane);
+  const int32_t gp = a.gp ? a.gp[group] : group_prefix32<32 / NREP>(a, t0, lane);
+  uint8_t* const stage = lds + wave * kStage;
+
+  auto merge = [&](const Segment& s, const Softmax& X) __attribute__((always_inline)) {
+    const float lt = X.l + __shfl_xor(X.l, 32, 64);
+    if (lane < 32) {
+      ms[wave][n] = X.m;
+      ls[wave][n] = lt;
+    }
+    __syncthreads();  // the states' maxima are known, and no wave stages any more
+    float M = ms[0][n];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = __builtin_fmaxf(M, ms[w][n]);
+    const float sc = X.m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(X.m - M);
+    // query n's 4 dims 4 u .. 4 u + 3 in 16-byte unit u ^ n of its 512 bytes
+    // (the 32 lanes of a write, and of a read below, on distinct units)
+    float4* const mine = reinterpret_cast<float4*>(lds) + wave * 1024 + n * 32;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int mt = i >> 2, j = i & 3, u = 8 * mt + 2 * j + h;
+      mine[u ^ n] = make_float4(X.O[mt][4 * j] * sc, X.O[mt][4 * j + 1] * sc, X.O[mt][4 * j + 2] * sc,
+                                X.O[mt][4 * j + 3] * sc);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = threadIdx.x; i < 1024; i += 64 * NW) {
+      const int qn = i >> 5, u = i & 31, tok = qn / NREP;
+      const int64_t t = t0 + tok;
+      float mx = ms[0][qn];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) mx = __builtin_fmaxf(mx, ms[w][qn]);
+      float L = 0.0f;
+      float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float4 x = reinterpret_cast<const float4*>(lds)[w * 1024 + qn * 32 + (u ^ qn)];
+        const float m = ms[w][qn];
+        L += m == -__builtin_inff() ? 0.0f : ls[w][qn] * __builtin_amdgcn_exp2f(m - mx);
+        acc.x += x.x;
+        acc.y += x.y;
+        acc.z += x.z;
+        acc.w += x.w;
+      }
+      const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+      if (t < a.T && tok >= s.first && tok < s.first + s.count) {
+        uint16_t* const op = a.out + t * a.sot + (kh * NREP + qn % NREP) * a.soh + 4 * u;
+        *reinterpret_cast<u32x2*>(op) =
+            u32x2{pack_bf16x2(acc.x * inv, acc.y * inv), pack_bf16x2(acc.z * inv, acc.w * inv)};
+      }
+    }
+  };
+
+  Softmax X;
+  bool nan = false;
+  if (gp > 0) {
+    const Segment s = whole_group<NREP>(a, gp, Q, lane);
+    attend_segment<NREP, false>(a, stage, kh, lane, Q, s, wave, NW, X, nan);
+    merge(s, X);
+    return;
+  }
+  const Segments<NREP> segs(a, t0, lane);
+  int single_until = 0;
+  for (int at = 0; at < segs.ntok;) {
+    if (threadIdx.x == 0) saw_nan = 0;
+    __syncthreads();  // the last merge has been read, the flag is clear
+    const Segment s = segs.next(at, Q, at < single_until);
+    nan = false;
+    attend_segment<NREP, true>(a, stage, kh, lane, Q, s, wave, NW, X, nan);
+    if (nan && lane == 0) saw_nan = 1;
+    __syncthreads();
+    if (saw_nan && s.count > 1) {
+      single_until = at + s.count;
+      __syncthreads();  // every wave has read the flag
+      continue;
+    }
+    merge(s, X);
+    at += s.count;
+  }
 }
 
 // Attention fused with the per-token e4m3 quant of its output (the o_proj
@@ -581,18 +663,24 @@ __global__ __launch_bounds__(256, 2) void paged_attn_grouped_d128(AttnArgs a) {
 // takes tokens w, w + 8, ...: the token's Hq x 128 bf16 values (4 heads per
 // pass, 8 dims per lane), row amax, scale = amax / 448 and the codes, in the
 // row kernels' arithmetic (quant8_e4m3).  The codes are bit-for-bit what
-// paged_attn_grouped_d128 followed by the per-token quant writes.
+// paged_attn_d128 followed by the per-token quant writes.
 template <int NREP>
 __global__ __launch_bounds__(512, 1) void paged_attn_grouped_quant_d128(AttnArgs a, uint8_t* qout, int64_t ldq,
                                                                         float* qscale) {
   constexpr int TOK = 32 / NREP;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[8 * 32 * kVRow];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[8 * kStage];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t group = blockIdx.x;
   const int64_t t0 = group * TOK;
   if (t0 >= a.T) return;
-  if (wave < a.Hk) grouped_item<NREP, true>(a, lds + wave * (32 * kVRow), group, wave, lane);
+  if (wave < a.Hk) {
+    u32x2 o[16];
+    attend_item<NREP>(a, lds + wave * kStage, group, wave, lane, o);
+    uint8_t* const op = lds + wave * kStage + (lane & 31) * kVRow;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) *reinterpret_cast<u32x2*>(op + 16 * i + 8 * (lane >> 5)) = o[i];
+  }
   __syncthreads();
   const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
   const int hq = static_cast<int>(a.Hq);
@@ -606,7 +694,7 @@ __global__ __launch_bounds__(512, 1) void paged_attn_grouped_quant_d128(AttnArgs
       const int head = 4 * p + hl;
       w[p] = u32x4{0, 0, 0, 0};
       if (head < hq) {
-        const uint8_t* src = lds + (head / NREP) * (32 * kVRow) + (tt * NREP + head % NREP) * kVRow + 2 * dl;
+        const uint8_t* src = lds + (head / NREP) * kStage + (tt * NREP + head % NREP) * kVRow + 2 * dl;
         w[p] = *reinterpret_cast<const u32x4*>(src);
       }
 #pragma unroll
@@ -637,42 +725,41 @@ __global__ __launch_bounds__(512, 1) void paged_attn_grouped_quant_d128(AttnArgs
   }
 }
 
-// The groups grouped_d128 leaves: one workgroup per group; its waves (8, or
-// 4 for 8-wide query groups, whose per-token registers need a whole SIMD
-// half) take the group's (token, kv head) pairs in turn, each on the VALU.
-template <int NREP>
-constexpr int token_waves() { return NREP >= 8 ? 4 : 8; }
-
-template <int NREP>
-__global__ __launch_bounds__(64 * token_waves<NREP>()) void paged_attn_tokens_d128(AttnArgs a) {
-  constexpr int TOK = 32 / NREP;
-  constexpr int NP = NREP >= 8 ? 1 : 16 / NREP;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * TOK;
-  if (t0 >= a.T) return;
-  if (a.gp ? a.gp[blockIdx.x] != 0 : group_shares_block<TOK>(a, t0, lane)) return;
-  const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
-  const int pairs = ntok * static_cast<int>(a.Hk);
-  for (int p = wave; p < pairs; p += token_waves<NREP>())
-  {
-    const int64_t t = t0 + p / a.Hk;
-    const int kh = static_cast<int>(p % a.Hk);
-    attend_token<NREP, NP>(a, t, kh, lane, a.out + t * a.sot + kh * NREP * a.soh, a.soh);
-  }
+// Waves per item for a launch of `items` whose slot lists hold `entries`
+// slots.  Items alone leave SIMDs idle below about 2048 (two waves on each of
+// 1024); splitting costs a merge and, in decode, the quant as a launch of its
+// own.  A prompt's tokens share one list (few entries a token); decode rows
+// each bring their own, so entries per token is their length.  Measured, us,
+// waves 1 / 2 / 4 / 8 (attention; the fused quant or the split plus quant for
+// decode; rows x keys, 16 query and 8 kv heads):
+//   50 x 202 (32 items)     22.6 /    - / 12.0 / 12.4
+//   512 x 130 (256)         17.9 / 13.8 / 12.6 / 12.9    512 x 1503   89.1 / - / 27.8 / 24.6
+//   1024 x 130 (512)        18.2 / 16.0 / 15.9 / 21.9    1024 x 1002  64.5 / 38.3 / 30.1 / 36.1
+//   1248 x 1133 (624)        180 / 98.9 / 73.4 / 75.4
+//   2048 x 130 (1024)       19.6 / 21.5 / 26.7 / 39.1    2048 x 1002  65.8 / 46.1 / 51.1 / 67.9
+//   4096 x 130 (2048)       21.9 /    - / 46.4 / 74.3    4096 x 1002  72.7 / 85.3 / 91.1 / 127
+//   prefill 1999 (1000)     76.9 / 47.9 / 44.5 / 60.3    4 x 500 (1000)  33.1 / 30.3 / 30.4 / 41.5
+//   prefill 4000 (2000)      159 /  122 /  125 /  159
+static int attn_waves(int64_t T, int64_t items, int64_t entries) {
+  const int64_t simds = 4 * num_cus();
+  const bool prompt = entries < 8 * T;
+  const int64_t keys = entries / T;
+  if (4 * items <= simds) return prompt || keys > 600 ? 8 : 4;
+  if (2 * items <= simds) return 4;
+  if (items <= simds) return prompt ? 4 : (keys < 300 ? 1 : (4 * items <= 3 * simds ? 4 : 2));
+  return prompt && items <= 2 * simds ? 2 : 1;
 }
 
-// One launch, or two for NREP >= 8 (the token path in a kernel of its own):
-// every group is taken by exactly one wave set.
 template <int NREP>
-static hipError_t launch_grouped(const AttnArgs& a, hipStream_t st) {
-  const int64_t groups = (a.T + 32 / NREP - 1) / (32 / NREP);
-  const int64_t items = groups * a.Hk;
-  hipLaunchKernelGGL((paged_attn_grouped_d128<NREP>), dim3(static_cast<unsigned>((items + 3) / 4)),
-                     dim3(256), 0, st, a);
-  if (kSeparateTokenKernel<NREP>)
-    hipLaunchKernelGGL((paged_attn_tokens_d128<NREP>), dim3(static_cast<unsigned>(groups)),
-                       dim3(64 * token_waves<NREP>()), 0, st, a);
+static hipError_t launch_attn(const AttnArgs& a, int waves, hipStream_t st) {
+  const int64_t items = (a.T + 32 / NREP - 1) / (32 / NREP) * a.Hk;
+  const dim3 grid(static_cast<unsigned>(items));
+  switch (waves) {
+    case 8: hipLaunchKernelGGL((paged_attn_split_d128<NREP, 8>), grid, dim3(512), 0, st, a); break;
+    case 4: hipLaunchKernelGGL((paged_attn_split_d128<NREP, 4>), grid, dim3(256), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((paged_attn_split_d128<NREP, 2>), grid, dim3(128), 0, st, a); break;
+    default: hipLaunchKernelGGL((paged_attn_d128<NREP>), grid, dim3(64), 0, st, a); break;
+  }
   return hipGetLastError();
 }
 
@@ -720,9 +807,39 @@ static int attn_args(AttnArgs& a, const void* q, int64_t sqt, int64_t sqh, const
   a.Hq = Hq;
   a.Hk = Hk;
   a.num_slots = num_slots;
+  a.row16 = skp == svp && skp > 0 && num_slots <= (int64_t(1) << 32) / (skp / 16) ? static_cast<uint32_t>(skp / 16) : 0;
   a.qscale = scale * 1.4426950408889634f;
   a.gp = group_prefix;
   return FR_OK;
+}
+
+extern "C" int fr_paged_attention_split_fp8(const void* q, int64_t sqt, int64_t sqh, const void* k_cache,
+                                            int64_t skp, int64_t skh, const void* v_cache, int64_t svp,
+                                            int64_t svh, int64_t num_slots, const int32_t* kv_indices,
+                                            const int32_t* kv_start, const int32_t* kv_len, void* out,
+                                            int64_t sot, int64_t soh, int64_t T, int64_t Hq, int64_t Hk,
+                                            int64_t D, float scale, const int32_t* group_prefix, int waves,
+                                            void* stream) {
+  AttnArgs a;
+  const int rc = attn_args(a, q, sqt, sqh, k_cache, skp, skh, v_cache, svp, svh, num_slots, kv_indices, kv_start,
+                           kv_len, T, Hq, Hk, D, scale, group_prefix);
+  if (rc != FR_OK) return rc;
+  if (waves != 1 && waves != 2 && waves != 4 && waves != 8) return FR_EINVAL;
+  if (T == 0) return FR_OK;
+  if (!out) return FR_EINVAL;
+  if ((reinterpret_cast<uintptr_t>(out) & 15u) || sot % 8 || soh % 8) return FR_EUNSUPPORTED;
+  a.out = static_cast<uint16_t*>(out);
+  a.sot = sot;
+  a.soh = soh;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipError_t e;
+  switch (Hq / Hk) {
+    case 1: e = launch_attn<1>(a, waves, st); break;
+    case 2: e = launch_attn<2>(a, waves, st); break;
+    case 4: e = launch_attn<4>(a, waves, st); break;
+    default: e = launch_attn<8>(a, waves, st); break;
+  }
+  return e == hipSuccess ? FR_OK : FR_ELAUNCH;
 }
 
 extern "C" int fr_paged_attention_fp8(const void* q, int64_t sqt, int64_t sqh, const void* k_cache,
@@ -732,24 +849,8 @@ extern "C" int fr_paged_attention_fp8(const void* q, int64_t sqt, int64_t sqh, c
                                       int64_t sot, int64_t soh, int64_t T, int64_t Hq, int64_t Hk,
                                       int64_t D, float scale, const int32_t* group_prefix,
                                       void* stream) {
-  AttnArgs a;
-  const int rc = attn_args(a, q, sqt, sqh, k_cache, skp, skh, v_cache, svp, svh, num_slots, kv_indices, kv_start,
-                           kv_len, T, Hq, Hk, D, scale, group_prefix);
-  if (rc != FR_OK) return rc;
-  if (T == 0) return FR_OK;
-  if (!out) return FR_EINVAL;
-  if ((reinterpret_cast<uintptr_t>(out) & 15u) || sot % 8 || soh % 8) return FR_EUNSUPPORTED;
-  a.out = static_cast<uint16_t*>(out);
-  a.sot = sot;
-  a.soh = soh;
-  hipError_t e;
-  switch (Hq / Hk) {
-    case 1: e = launch_grouped<1>(a, static_cast<hipStream_t>(stream)); break;
-    case 2: e = launch_grouped<2>(a, static_cast<hipStream_t>(stream)); break;
-    case 4: e = launch_grouped<4>(a, static_cast<hipStream_t>(stream)); break;
-    default: e = launch_grouped<8>(a, static_cast<hipStream_t>(stream)); break;
-  }
-  return e == hipSuccess ? FR_OK : FR_ELAUNCH;
+  return fr_paged_attention_split_fp8(q, sqt, sqh, k_cache, skp, skh, v_cache, svp, svh, num_slots, kv_indices,
+                                      kv_start, kv_len, out, sot, soh, T, Hq, Hk, D, scale, group_prefix, 1, stream);
 }
 
 extern "C" int fr_paged_attention_quant_fp8(const void* q, int64_t sqt, int64_t sqh, const void* k_cache,
@@ -785,6 +886,11 @@ extern "C" int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t H
   if (nrep != 1 && nrep != 2 && nrep != 4 && nrep != 8) return -1;
   const int64_t tok = 32 / nrep;
   return (T + tok - 1) / tok;
+}
+
+extern "C" int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries) {
+  const int64_t groups = fr_paged_attention_plan_size(T, Hq, Hk);
+  return groups <= 0 || entries < 0 ? 1 : attn_waves(T, groups * Hk, entries);
 }
 
 extern "C" int fr_paged_attention_plan(const int32_t* kv_indices, const int32_t* kv_start,

@@ -258,6 +258,22 @@ int fr_paged_attention_quant_fp8(const void* q, int64_t sqt, int64_t sqh, const 
                                  int64_t Hq, int64_t Hk, int64_t D, float scale,
                                  const int32_t* group_prefix, void* stream);
 
+/* fr_paged_attention_fp8 with the keys of each item (one query group and kv
+ * head) split over `waves` waves of a workgroup (1, 2, 4 or 8; 1 is
+ * fr_paged_attention_fp8), for launches whose items alone do not fill the
+ * chip.  The partial sums are merged in a fixed order, another one than
+ * unsplit: rows may differ from it in the last bf16 bit. */
+int fr_paged_attention_split_fp8(const void* q, int64_t sqt, int64_t sqh, const void* k_cache,
+                                 int64_t skp, int64_t skh, const void* v_cache, int64_t svp, int64_t svh,
+                                 int64_t num_slots, const int32_t* kv_indices, const int32_t* kv_start,
+                                 const int32_t* kv_len, void* out, int64_t sot, int64_t soh, int64_t T,
+                                 int64_t Hq, int64_t Hk, int64_t D, float scale,
+                                 const int32_t* group_prefix, int waves, void* stream);
+
+/* The number of waves that suits T tokens whose lists hold `entries` slots
+ * together (the length of kv_indices). */
+int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries);
+
 /* The per-batch attention plan, computed once for all layers that attend
  * over the same kv_indices / kv_start / kv_len: for each group of 32 / (Hq /
  * Hk) consecutive query tokens, the slot prefix all of them share, rounded
