@@ -220,7 +220,7 @@ def _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len):
     if k_cache.dtype != torch.float8_e4m3fn or v_cache.dtype != torch.float8_e4m3fn:
         raise TypeError("paged_attention reads an e4m3 KV pool")
     for t in (kv_indices, kv_start, kv_len):
-        if t.dtype != torch.int32 or not t.is_contiguous():
+        if t.dtype is not torch.int32 or not t.is_contiguous():
             raise TypeError("kv_indices / kv_start / kv_len must be contiguous int32")
     T, Hq, D = q.shape
     slots, Hk, Dk = k_cache.shape

@@ -11,7 +11,14 @@ from __future__ import annotations
 
 import torch
 
-from flashrec_amd._lib import Unsupported, call, require_device, stream_of
+from flashrec_amd._lib import Unsupported, as_vector, call, require_device, stream_of
+
+
+def _first(x: torch.Tensor, t: int) -> torch.Tensor:
+    """The first ``t`` values as contiguous int64 (``x`` itself where it is that)."""
+    if x.dtype is torch.int64 and x.dim() == 1 and x.shape[0] == t and x.is_contiguous():
+        return x
+    return x.view(-1)[:t].to(dtype=torch.int64).contiguous()
 
 
 @torch.compiler.disable
@@ -64,11 +71,13 @@ def fused_qk_norm_rope_store_fp8(
         k = k.contiguous()
     if v.stride(-1) != 1:
         v = v.contiguous()
-    pos = positions.view(-1)[:t].to(dtype=torch.int64).contiguous()
-    loc64 = loc.view(-1)[:t].to(dtype=torch.int64).contiguous()
-    qw = q_weight.reshape(-1).to(device=q.device, dtype=torch.bfloat16).contiguous()
-    kw = k_weight.reshape(-1).to(device=q.device, dtype=torch.bfloat16).contiguous()
-    cs = cos_sin_cache.to(device=q.device, dtype=torch.float32).contiguous()
+    pos = _first(positions, t)
+    loc64 = _first(loc, t)
+    qw = as_vector(q_weight, torch.bfloat16, q)
+    kw = as_vector(k_weight, torch.bfloat16, q)
+    cs = cos_sin_cache
+    if cs.dtype is not torch.float32 or cs.get_device() != q.get_device() or not cs.is_contiguous():
+        cs = cs.to(device=q.device, dtype=torch.float32).contiguous()
     if int(qw.numel()) != d or int(kw.numel()) != d:
         return False
     try:

@@ -14,7 +14,7 @@ from typing import Optional
 
 import torch
 
-from flashrec_amd._lib import DTYPE_CODE, call, require_device, stream_of
+from flashrec_amd._lib import DTYPE_CODE, as_rows, as_vector, call, require_device, stream_of
 from flashrec_amd.kernel.sglops import _ACT
 
 _FP8_MAX = 448.0
@@ -31,14 +31,14 @@ def _launch(
     require_device(x, residual)
     orig = x.shape
     hidden = int(weight.numel())
-    x2 = x.reshape(-1, hidden).contiguous()
+    x2 = as_rows(x, hidden)
     # the norm weight in the activations' dtype, as the reference's fused
     # path passes it (rms_fp8.py:86)
-    w = weight.reshape(-1).to(device=x.device, dtype=x.dtype).contiguous()
+    w = as_vector(weight, x.dtype, x)
     rows = int(x2.shape[0])
     r2 = None
     if residual is not None:
-        r2 = residual.reshape(-1, hidden).contiguous()
+        r2 = as_rows(residual, hidden)
         if r2.shape != x2.shape:
             raise ValueError(f"residual {tuple(residual.shape)} does not match x {tuple(orig)}")
     y = torch.empty(x2.shape, dtype=torch.float8_e4m3fn, device=x2.device)
@@ -46,7 +46,7 @@ def _launch(
     call("fr_rms_quant_fp8", x2.data_ptr(), DTYPE_CODE[x.dtype], x2.stride(0),
          None if r2 is None else r2.data_ptr(), 0 if r2 is None else r2.stride(0),
          w.data_ptr(), rows, hidden, float(eps), y.data_ptr(), scale.data_ptr(), stream_of(x))
-    res_out = r2.reshape(residual.shape) if r2 is not None else None
+    res_out = r2.reshape(residual.shape) if r2 is not None and r2 is not residual else r2
     return y, scale, res_out
 
 

@@ -13,7 +13,7 @@ from typing import NamedTuple, Optional
 
 import torch
 
-from flashrec_amd._lib import DTYPE_CODE, call, load, ptr, require_device, stream_of
+from flashrec_amd._lib import DTYPE_CODE, as_vector, call, load, ptr, require_device, stream_of
 
 _FP8_MAX = 448.0
 
@@ -27,12 +27,12 @@ _ACT = (torch.bfloat16, torch.float16, torch.float32)
 
 def _vec(weight: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """The norm weight as a contiguous vector in the activations' dtype."""
-    return weight.reshape(-1).to(device=x.device, dtype=x.dtype).contiguous()
+    return as_vector(weight, x.dtype, x)
 
 
 def _rows(x: torch.Tensor, width: int) -> torch.Tensor:
     """[..., width] -> [rows, width] with unit inner stride (copy only if needed)."""
-    x2 = x.reshape(-1, width)
+    x2 = x if x.dim() == 2 and x.shape[1] == width else x.reshape(-1, width)
     if x2.stride(-1) != 1 or (x2.shape[0] > 1 and x2.stride(0) < width):
         x2 = x2.contiguous()
     return x2
@@ -194,8 +194,8 @@ def fp8_scaled_mm(
     if not (b.stride(0) == 1 and (n <= 1 or b.stride(1) >= k)):
         b = b.t().contiguous().t()  # column-major copy
     a, b, k = _mfma_operands(a, b, m, n, k)
-    sa = scale_a.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
-    sb = scale_b.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
+    sa = as_vector(scale_a, torch.float32, a)
+    sb = as_vector(scale_b, torch.float32, a)
     if sa.numel() not in (1, m) or sb.numel() not in (1, n):
         raise ValueError("scale_a must have 1 or M values and scale_b 1 or N values")
     bias_t = None
@@ -246,8 +246,8 @@ def fp8_scaled_mm_residual(
     if not (b.stride(0) == 1 and (n <= 1 or b.stride(1) >= k)):
         b = b.t().contiguous().t()
     a, b, k = _mfma_operands(a, b, m, n, k)
-    sa = scale_a.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
-    sb = scale_b.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
+    sa = as_vector(scale_a, torch.float32, a)
+    sb = as_vector(scale_b, torch.float32, a)
     if sa.numel() not in (1, m) or sb.numel() not in (1, n):
         raise ValueError("scale_a must have 1 or M values and scale_b 1 or N values")
     lda = a.stride(0) if m > 1 else k
@@ -342,8 +342,8 @@ def fp8_scaled_mm_prearranged(
         a16 = torch.zeros((m, k16), dtype=torch.uint8, device=a.device)
         a16[:, :k] = a.view(torch.uint8)
         a, k, lda = a16.view(a_fp8.dtype), k16, k16
-    sa = scale_a.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
-    sb = scale_b.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
+    sa = as_vector(scale_a, torch.float32, a)
+    sb = as_vector(scale_b, torch.float32, a)
     if sa.numel() not in (1, m) or sb.numel() not in (1, n):
         raise ValueError("scale_a must have 1 or M values and scale_b 1 or N values")
     ldr = 0 if residual is None else (residual.stride(0) if m > 1 else n)
@@ -403,8 +403,8 @@ def fp8_scaled_mm_silu(
     if not (b.stride(0) == 1 and (n <= 1 or b.stride(1) >= k)):
         b = b.t().contiguous().t()
     a, b, k = _mfma_operands(a, b, m, n, k)
-    sa = scale_a.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
-    sb = scale_b.reshape(-1).to(device=a.device, dtype=torch.float32).contiguous()
+    sa = as_vector(scale_a, torch.float32, a)
+    sb = as_vector(scale_b, torch.float32, a)
     if sa.numel() not in (1, m) or sb.numel() not in (1, n):
         raise ValueError("scale_a must have 1 or M values and scale_b 1 or N values")
     lda = a.stride(0) if m > 1 else k

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from flashrec_amd._lib import DTYPE_CODE, call, require_device, stream_of
+from flashrec_amd._lib import DTYPE_CODE, as_rows, call, require_device, stream_of
 from flashrec_amd.kernel.sglops import _ACT
 
 _FP8_MAX = 448.0
@@ -28,7 +28,7 @@ def silu_and_mul_per_token_quant_fp8(
     if last % 2 != 0:
         raise ValueError("silu_and_mul_per_token_quant_fp8 needs an even last dimension")
     d = last // 2
-    x2 = x.reshape(-1, last).contiguous()
+    x2 = as_rows(x, last)
     rows = int(x2.shape[0])
     y = torch.empty((rows, d), dtype=torch.float8_e4m3fn, device=x2.device)
     scale = torch.empty((rows, 1), dtype=torch.float32, device=x2.device)

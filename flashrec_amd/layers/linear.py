@@ -113,9 +113,9 @@ class Linear(nn.Module):
     def _prearranged(self) -> PrearrangedFp8Weight:
         """The codes in the prearranged GEMM's layout, built when first needed
         on the codes' device (and kept until the weights change or move)."""
-        cached = self.__dict__.get("_pre")
-        if cached is None or cached.data.device != self.w_codes.device:
-            cached = prearrange_fp8_weight(self.w_codes.t())
+        cached, codes = self.__dict__.get("_pre"), self._buffers["w_codes"]
+        if cached is None or cached.data.get_device() != codes.get_device():
+            cached = prearrange_fp8_weight(codes.t())
             self.__dict__["_pre"] = cached
         return cached
 
@@ -205,17 +205,19 @@ class Linear(nn.Module):
         """GEMM of already quantised ``[M, K]`` e4m3 rows with their ``[M, 1]``
         scales; the result has shape ``orig_shape[:-1] + (out_features,)``
         (linear.py:134-142, 153-172)."""
-        if self.w_codes is None:
+        # read from the module's dicts: each attribute lookup through
+        # Module.__getattr__ costs most of a microsecond
+        codes, scale, bias = self._buffers["w_codes"], self._buffers["w_scale"], self.bias
+        if codes is None:
             raise RuntimeError("Linear.forward_fp8 needs fp8 weights (load an fp8 checkpoint "
                                "or pass quantize_fp8=True)")
-        if self.w_codes.device != q.device:
-            raise ValueError(f"activations on {q.device}, fp8 weights on {self.w_codes.device}: "
+        if codes.get_device() != q.get_device():
+            raise ValueError(f"activations on {q.device}, fp8 weights on {codes.device}: "
                              "move the module with .to() first")
-        if self.bias is None:
-            out = fp8_scaled_mm_prearranged(q, self._prearranged(), a_scale, self.w_scale, out_dtype)
+        if bias is None:
+            out = fp8_scaled_mm_prearranged(q, self._prearranged(), a_scale, scale, out_dtype)
         else:
-            out = fp8_scaled_mm(q, self.w_codes.t(), a_scale, self.w_scale, out_dtype,
-                                self.bias.to(dtype=out_dtype))
+            out = fp8_scaled_mm(q, codes.t(), a_scale, scale, out_dtype, bias.to(dtype=out_dtype))
         return out.view(*tuple(orig_shape)[:-1], self.out_features)
 
     def forward_fp8_residual(self, q: torch.Tensor, a_scale: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
