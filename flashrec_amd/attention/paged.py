@@ -176,7 +176,8 @@ class AttentionBackend:
 
 
 def plan_size(T: int, hq: int, hk: int) -> int:
-    """Entries of an attention plan for T query tokens (groups of 32 / (hq / hk))."""
+    """Entries of an attention plan for T query tokens: one per group of 32 /
+    (hq / hk) of them, then two per token."""
     n = int(load().fr_paged_attention_plan_size(int(T), int(hq), int(hk)))
     if n < 0:
         raise ValueError(f"unsupported head ratio {hq}/{hk}")
@@ -186,8 +187,9 @@ def plan_size(T: int, hq: int, hk: int) -> int:
 def attention_plan(kv_indices: torch.Tensor, kv_start: torch.Tensor, kv_len: torch.Tensor,
                    hq: int, hk: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The shared slot prefix (rounded down to 32) of each group of 32 / (hq /
-    hk) consecutive query tokens: computed once per batch, passed to every
-    layer's ``paged_attention`` as ``group_prefix``."""
+    hk) consecutive query tokens, then the kernels' own entries (how a group's
+    tokens fall into runs with common keys): computed once per batch, passed
+    to every layer's ``paged_attention`` as ``group_prefix``."""
     require_device(kv_indices, kv_start, kv_len)
     T = int(kv_start.numel())
     n = plan_size(T, hq, hk)

@@ -43,7 +43,7 @@ struct AttnArgs {
   int64_t T, Hq, Hk, num_slots;
   uint32_t row16;  // slot stride of both caches in 16-byte units, 0 where they differ or offsets pass 2^32
   float qscale;  // softmax scale * log2(e)
-  const int32_t* gp;  // [groups] slot prefix a group's tokens share, rounded down to 32, or null
+  const int32_t* gp;  // the plan (attn_group_plan), or null
 };
 
 // Longest slot prefix shared by the `count` tokens from t0 on (count <= TOK).
@@ -86,13 +86,6 @@ __device__ __forceinline__ int32_t tokens_prefix(const AttnArgs& a, int64_t t0, 
   return min(P, lenmin);
 }
 
-// The slot prefix shared by a whole group, rounded down to 32 (the plan's
-// entry).
-template <int TOK>
-__device__ __forceinline__ int32_t group_prefix32(const AttnArgs& a, int64_t t0, int lane) {
-  return tokens_prefix<TOK>(a, t0, static_cast<int>(min<int64_t>(TOK, a.T - t0)), lane) & ~31;
-}
-
 // Bit tt (1 .. count-1): token t0 + tt reads the slot list of token t0 + tt -
 // 1, or shares at least its first 32 slots.
 template <int TOK>
@@ -121,16 +114,6 @@ __device__ __forceinline__ uint32_t linked_tokens(const AttnArgs& a, int64_t t0,
   for (int tt = 1; tt < TOK; ++tt)
     if (((tryit >> tt) & 1u) && __ballot(x[tt] != y[tt]) == 0) linked |= 1u << tt;
   return linked;
-}
-
-// The plan: one wave per group, the group's shared prefix for every layer.
-template <int TOK>
-__global__ __launch_bounds__(256) void attn_group_plan(AttnArgs a, int32_t* gp, int64_t groups) {
-  const int lane = threadIdx.x & 63;
-  const int64_t group = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (group >= groups) return;
-  const int32_t p = group_prefix32<TOK>(a, group * TOK, lane);
-  if (lane == 0) gp[group] = p;
 }
 
 // ---------------------------------------------------------------------------
@@ -436,63 +419,119 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, uint8_t* stage
   }
 }
 
-// The segments of a group whose tokens do not all share 32 slots, in token
-// order: next() gives the one that starts at token `at`.
-template <int NREP>
-struct Segments {
-  static constexpr int TOK = 32 / NREP;
-  const AttnArgs& a;
-  int64_t t0;
-  int lane, ntok;
-  uint32_t linked;
-  __device__ __forceinline__ Segments(const AttnArgs& a_, int64_t t0_, int lane_)
-      : a(a_), t0(t0_), lane(lane_), ntok(static_cast<int>(min<int64_t>(TOK, a_.T - t0_))) {
-    linked = linked_tokens<TOK>(a, t0, ntok, lane);
-  }
-  __device__ __forceinline__ Segment next(int at, const Query& Q, bool single) const {
-    Segment s{at, 1, 0, true};
-    if (single) return s;
-    while (at + s.count < ntok && ((linked >> (at + s.count)) & 1u)) ++s.count;
-    // one list for all of them?
-    const int32_t st = __builtin_amdgcn_readlane(Q.start, at * NREP);
-    const int tok = (lane & 31) / NREP;
-    const bool other = tok >= at && tok < at + s.count && Q.start != st;
-    if (__ballot(other) == 0) return s;
-    s.one_list = false;
-    s.shared = tokens_prefix<TOK>(a, t0 + at, s.count, lane);
-    return s;
-  }
-};
-
 // The whole group as one segment, from its shared prefix rounded down to 32:
 // the up to 31 shared positions past that join the common blocks (as own rows
 // they would take NREP keys a block: at 28 of them 14 blocks instead of one).
-template <int NREP>
-__device__ __forceinline__ Segment whole_group(const AttnArgs& a, int32_t p32, const Query& Q, int lane) {
-  constexpr int TOK = 32 / NREP;
-  const int32_t st = __builtin_amdgcn_readfirstlane(Q.start);
-  if (__ballot(Q.ok && Q.start != st) == 0) return Segment{0, TOK, p32, true};
-  int32_t minlen = Q.ok ? Q.len : 0x7FFFFFFF, maxlen = Q.len;
+// Lane stride * tt holds token tt's list start and length in (start, len).
+template <int TOK>
+__device__ __forceinline__ Segment whole_group(const AttnArgs& a, int32_t p32, int32_t start, int32_t len, bool ok,
+                                               int stride, int lane) {
+  const int32_t st = __builtin_amdgcn_readfirstlane(start);
+  if (__ballot(ok && start != st) == 0) return Segment{0, TOK, p32, true};
+  int32_t minlen = ok ? len : 0x7FFFFFFF;
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    minlen = min(minlen, __shfl_xor(minlen, o, 64));
-    maxlen = max(maxlen, __shfl_xor(maxlen, o, 64));
-  }
-  // at most two own blocks in any case: the look costs as much as they do
-  if (maxlen - p32 <= 2 * NREP) return Segment{0, TOK, p32, false};
+  for (int o = 32; o >= 1; o >>= 1) minlen = min(minlen, __shfl_xor(minlen, o, 64));
   // (every list holds p32 positions and more; a token past the last one
-  // repeats the first: Q.start)
+  // repeats the first)
   const bool in = p32 + (lane & 31) < minlen;
   const int32_t pos = in ? p32 + (lane & 31) : 0;
   int32_t sv[TOK];
 #pragma unroll
-  for (int tt = 0; tt < TOK; ++tt) sv[tt] = a.kv_indices[__builtin_amdgcn_readlane(Q.start, tt * NREP) + pos];
-  bool ok = in;
+  for (int tt = 0; tt < TOK; ++tt) sv[tt] = a.kv_indices[__builtin_amdgcn_readlane(start, tt * stride) + pos];
+  bool same = in;
 #pragma unroll
-  for (int tt = 1; tt < TOK; ++tt) ok = ok && sv[tt] == sv[0];
-  const uint32_t bad = static_cast<uint32_t>(__ballot(!ok));  // the two halves agree
+  for (int tt = 1; tt < TOK; ++tt) same = same && sv[tt] == sv[0];
+  const uint32_t bad = static_cast<uint32_t>(__ballot(!same));  // the two halves agree
   return Segment{0, TOK, p32 + (bad ? __builtin_ctz(bad) : 32), false};
 }
+
+// The segment of a group that starts at token `at`, for groups whose tokens do
+// not all share 32 slots: the run of linked tokens from there on.  Lane layout
+// of (tok, start) as above.
+template <int TOK>
+__device__ __forceinline__ Segment next_segment(const AttnArgs& a, int64_t t0, int ntok, uint32_t linked, int at,
+                                                int tok, int32_t start, int stride, int lane) {
+  Segment s{at, 1, 0, true};
+  while (at + s.count < ntok && ((linked >> (at + s.count)) & 1u)) ++s.count;
+  // one list for all of them?
+  const int32_t st = __builtin_amdgcn_readlane(start, at * stride);
+  if (__ballot(tok >= at && tok < at + s.count && start != st) == 0) return s;
+  s.one_list = false;
+  s.shared = tokens_prefix<TOK>(a, t0 + at, s.count, lane);
+  return s;
+}
+
+// The plan, one wave per group, made once for every layer of a batch (entries
+// in fr_paged_attention_plan_size's order): the group's shared prefix rounded
+// down to 32; then for every token that starts a segment the number of its
+// tokens, negative where they read one list (0: the token continues one);
+// then the segments' shared prefixes.
+template <int TOK>
+__global__ __launch_bounds__(256) void attn_group_plan(AttnArgs a, int32_t* gp, int64_t groups) {
+  const int lane = threadIdx.x & 63;
+  const int64_t group = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (group >= groups) return;
+  const int64_t t0 = group * TOK;
+  const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
+  const bool ok = lane < ntok;
+  const int32_t start = a.kv_start[ok ? t0 + lane : t0], len = a.kv_len[ok ? t0 + lane : t0];
+  const int32_t p = tokens_prefix<TOK>(a, t0, ntok, lane);
+  if (lane == 0) gp[group] = p & ~31;
+  int32_t cnt = 0, sh = 0;  // lane tt: token t0 + tt's entries
+  if (p >= 32) {
+    const int32_t st = __builtin_amdgcn_readfirstlane(start);
+    const bool one = __ballot(ok && start != st) == 0;
+    cnt = lane == 0 ? (one ? -ntok : ntok) : 0;
+    sh = lane == 0 ? p : 0;
+  } else {
+    const uint32_t linked = linked_tokens<TOK>(a, t0, ntok, lane);
+    for (int at = 0; at < ntok;) {
+      const Segment s = next_segment<TOK>(a, t0, ntok, linked, at, ok ? lane : TOK, start, 1, lane);
+      if (lane == at) {
+        cnt = s.one_list ? -s.count : s.count;
+        sh = s.shared;
+      }
+      at += s.count;
+    }
+  }
+  if (ok) {
+    gp[groups + t0 + lane] = cnt;
+    gp[groups + a.T + t0 + lane] = sh;
+  }
+}
+
+// A group's segments: from the plan, or found here.
+template <int NREP>
+struct Segments {
+  static constexpr int TOK = 32 / NREP;
+  int64_t t0;
+  int ntok;
+  int32_t whole;  // prefix shared by the whole group rounded down to 32 (0: several segments)
+  int32_t cnt = 0, sh = 0;  // lane tt: the plan's entries of token t0 + tt
+  uint32_t linked = 0;
+  __device__ __forceinline__ Segments(const AttnArgs& a, int64_t t0_, int64_t group, int lane)
+      : t0(t0_), ntok(static_cast<int>(min<int64_t>(TOK, a.T - t0_))) {
+    if (a.gp) {
+      const int64_t groups = (a.T + TOK - 1) / TOK;
+      const int32_t* const e = a.gp + groups + t0 + (lane < ntok ? lane : 0);
+      whole = a.gp[group];
+      cnt = e[0];
+      sh = e[a.T];
+    } else {
+      whole = tokens_prefix<TOK>(a, t0, ntok, lane) & ~31;
+      if (whole == 0) linked = linked_tokens<TOK>(a, t0, ntok, lane);
+    }
+  }
+  __device__ __forceinline__ Segment at(const AttnArgs& a, int first, const Query& Q, bool single, int lane) const {
+    if (single) return Segment{first, 1, 0, true};
+    if (a.gp) {
+      const int32_t c = __builtin_amdgcn_readlane(cnt, first);
+      return Segment{first, c < 0 ? -c : c, __builtin_amdgcn_readlane(sh, first), c < 0};
+    }
+    if (whole > 0) return whole_group<TOK>(a, whole, Q.start, Q.len, Q.ok, NREP, lane);
+    return next_segment<TOK>(a, t0, ntok, linked, first, (lane & 31) / NREP, Q.start, NREP, lane);
+  }
+};
 
 // A lane's normalised output row piece: 4 consecutive dims 32 mt + 8 j + 4 h ..
 // as bf16 (no visible key: zeros, the softmax of an empty row is undefined).
@@ -507,22 +546,21 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, uint8_t* stage, i
                                             u32x2 (&o)[16]) {
   const int64_t t0 = group * (32 / NREP);
   const Query Q = load_query<NREP>(a, t0, kh, lane);
-  const int32_t gp = a.gp ? a.gp[group] : group_prefix32<32 / NREP>(a, t0, lane);
+  const Segments<NREP> segs(a, t0, group, lane);
   Softmax X;
   bool nan = false;
-  if (gp > 0) {
-    attend_segment<NREP, false>(a, stage, kh, lane, Q, whole_group<NREP>(a, gp, Q, lane), 0, 1, X, nan);
+  if (segs.whole > 0) {
+    attend_segment<NREP, false>(a, stage, kh, lane, Q, segs.at(a, 0, Q, false, lane), 0, 1, X, nan);
     const float lt = X.l + __shfl_xor(X.l, 32, 64);
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[i] = out4(X, inv, i >> 2, i & 3);
     return;
   }
-  const Segments<NREP> segs(a, t0, lane);
   const int tok = (lane & 31) / NREP;
   int single_until = 0;
   for (int at = 0; at < segs.ntok;) {
-    const Segment s = segs.next(at, Q, at < single_until);
+    const Segment s = segs.at(a, at, Q, at < single_until, lane);
     nan = false;
     attend_segment<NREP, true>(a, stage, kh, lane, Q, s, 0, 1, X, nan);
     if (nan && s.count > 1) {
@@ -576,7 +614,7 @@ __global__ __launch_bounds__(64 * NW, 2) void paged_attn_split_d128(AttnArgs a) 
   const int64_t t0 = group * (32 / NREP);
   const int n = lane & 31, h = lane >> 5;
   const Query Q = load_query<NREP>(a, t0, kh, lane);
-  const int32_t gp = a.gp ? a.gp[group] : group_prefix32<32 / NREP>(a, t0, lane);
+  const Segments<NREP> segs(a, t0, group, lane);
   uint8_t* const stage = lds + wave * kStage;
 
   auto merge = [&](const Segment& s, const Softmax& X) __attribute__((always_inline)) {
@@ -630,18 +668,17 @@ __global__ __launch_bounds__(64 * NW, 2) void paged_attn_split_d128(AttnArgs a) 
 
   Softmax X;
   bool nan = false;
-  if (gp > 0) {
-    const Segment s = whole_group<NREP>(a, gp, Q, lane);
+  if (segs.whole > 0) {
+    const Segment s = segs.at(a, 0, Q, false, lane);
     attend_segment<NREP, false>(a, stage, kh, lane, Q, s, wave, NW, X, nan);
     merge(s, X);
     return;
   }
-  const Segments<NREP> segs(a, t0, lane);
   int single_until = 0;
   for (int at = 0; at < segs.ntok;) {
     if (threadIdx.x == 0) saw_nan = 0;
     __syncthreads();  // the last merge has been read, the flag is clear
-    const Segment s = segs.next(at, Q, at < single_until);
+    const Segment s = segs.at(a, at, Q, at < single_until, lane);
     nan = false;
     attend_segment<NREP, true>(a, stage, kh, lane, Q, s, wave, NW, X, nan);
     if (nan && lane == 0) saw_nan = 1;
@@ -880,7 +917,8 @@ extern "C" int fr_paged_attention_quant_fp8(const void* q, int64_t sqt, int64_t 
   return e == hipSuccess ? FR_OK : FR_ELAUNCH;
 }
 
-extern "C" int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t Hk) {
+// Query groups of T tokens (-1: unsupported head ratio).
+static int64_t attn_groups(int64_t T, int64_t Hq, int64_t Hk) {
   if (T < 0 || Hq <= 0 || Hk <= 0 || Hq % Hk != 0) return -1;
   const int64_t nrep = Hq / Hk;
   if (nrep != 1 && nrep != 2 && nrep != 4 && nrep != 8) return -1;
@@ -888,15 +926,20 @@ extern "C" int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t H
   return (T + tok - 1) / tok;
 }
 
+extern "C" int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t Hk) {
+  const int64_t groups = attn_groups(T, Hq, Hk);
+  return groups < 0 ? -1 : groups + 2 * T;
+}
+
 extern "C" int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries) {
-  const int64_t groups = fr_paged_attention_plan_size(T, Hq, Hk);
+  const int64_t groups = attn_groups(T, Hq, Hk);
   return groups <= 0 || entries < 0 ? 1 : attn_waves(T, groups * Hk, entries);
 }
 
 extern "C" int fr_paged_attention_plan(const int32_t* kv_indices, const int32_t* kv_start,
                                        const int32_t* kv_len, int64_t T, int64_t Hq, int64_t Hk,
                                        int32_t* group_prefix, void* stream) {
-  const int64_t groups = fr_paged_attention_plan_size(T, Hq, Hk);
+  const int64_t groups = attn_groups(T, Hq, Hk);
   if (groups < 0) return FR_EUNSUPPORTED;
   if (groups == 0) return FR_OK;
   if (!kv_indices || !kv_start || !kv_len || !group_prefix) return FR_EINVAL;

@@ -277,7 +277,9 @@ int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries)
 /* The per-batch attention plan, computed once for all layers that attend
  * over the same kv_indices / kv_start / kv_len: for each group of 32 / (Hq /
  * Hk) consecutive query tokens, the slot prefix all of them share, rounded
- * down to 32 (0: none).  fr_paged_attention_plan_size gives the entry count
+ * down to 32 (0: none); after these, for the attention kernels, how each
+ * group's tokens fall into runs with common keys.  fr_paged_attention_plan_size
+ * gives the entry count
  * (-1 for an unsupported head ratio).  Passing the plan as group_prefix to
  * fr_paged_attention_fp8 skips that detection in every call (null: each call
  * detects it).  No counterpart in the reference: flashinfer plans its own
