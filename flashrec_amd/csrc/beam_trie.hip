@@ -16,21 +16,26 @@
 // else next_node[node][tok - token_base].  NaN scores are treated as masked.
 //
 // Layout for MI355X.  Per request the candidates are BW beams x C columns,
-// each beam's C already sorted descending (they come from a per-row sorted
-// top-k), so the top K is a merge.  A candidate is one 64-bit key: the
-// orderable bits of its score in the high word, the complement of its flat
-// index in the low word, so "larger key" is exactly the ranking above and
-// every merge is exact.
+// each beam's C sorted descending (they come from a per-row sorted top-k).  A
+// candidate is one 64-bit key: the orderable bits of its score in the high
+// word, the complement of its flat index in the low word, so keys are distinct
+// and "larger key" is exactly the ranking above.  Both kernels are a chain of
+// latencies (one request's beam step takes as long as eight requests'), so
+// they select instead of merging: a 2048-bin LDS histogram of the key range,
+// narrowed to the bin that holds the K-th key until few enough keys are left
+// (select_top), is a handful of barriers where a tree of pairwise merges was
+// a binary search and a walk of dependent LDS reads per level.
 //   kernel 1, one workgroup per (request, slice of BS beams): each wave
-//     compacts its beams' valid candidates into per-beam sorted lists of at
-//     most K keys (ballot prefix sums; stops at K), then the BS lists are
-//     merged pairwise in LDS (merge path: each output finds its split by a
-//     binary search, all outputs in parallel, one barrier per tree level)
-//     into the slice's top K, written to the caller's scratch;
-//   kernel 2, one workgroup per request: merges the slices' lists the same
-//     way (in groups that fit LDS, each folded into a running top K), writes
-//     vals / parents / tokens / indices, then the expanded token rows and the
-//     advanced trie nodes.
+//     compacts its beams' valid candidates into per-beam lists of at most K
+//     keys (ballot prefix sums; stops at K); the slice's best K of them, in
+//     no particular order, go to the caller's scratch;
+//   kernel 2, one workgroup per request: selects at most 1024 keys that hold
+//     the top K from the slices' lists, sorts them (one key per thread),
+//     writes vals / parents / tokens / indices, then the expanded token rows
+//     and the advanced trie nodes.
+// 8 x 512 beams x 1024 candidates -> top 512: 34.0 + 33.6 us with merge trees,
+// 18.2 + 18.3 so; 1 x 512 33.6 + 33.7 -> 15.4 + 17.8; 8 x 35 21.4 + 10.6 -> 10.1
+// + 8.4.  What is left is latency: kernel 2 is one CU per request.
 #include <mutex>
 
 #include "fr_common.h"
@@ -76,197 +81,356 @@ __device__ __forceinline__ uint64_t make_key(float v, uint32_t idx) {
 __device__ __forceinline__ float key_val(uint64_t k) { return from_order_bits(static_cast<uint32_t>(k >> 32)); }
 __device__ __forceinline__ uint32_t key_idx(uint64_t k) { return ~static_cast<uint32_t>(k); }
 
-__device__ __forceinline__ bool cand_ok(const GenrecArgs& a, int64_t node, int64_t t) {
-  if (node < 0) return true;
-  const int64_t rel = t - a.token_base;
-  if (rel < 0 || rel >= a.vsz || a.n_nodes <= 0) return false;
-  const int64_t safe = node < 0 ? 0 : (node > a.n_nodes - 1 ? a.n_nodes - 1 : node);
-  return a.allow[safe * a.vsz + rel] != 0;
+constexpr int kBins = 2048;  // select_top's histogram
+
+// LDS of select_top.
+struct SelectLds {
+  uint32_t hist[kBins];
+  uint32_t wsum[16];
+  uint64_t hi[16], lo[16];
+  uint64_t edge[2];  // bin of the K-th key, keys before it
+  uint32_t at;       // keys in it
+};
+
+__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
+  const uint32_t lo = __shfl_xor(static_cast<uint32_t>(v), m, 64);
+  const uint32_t hi = __shfl_xor(static_cast<uint32_t>(v >> 32), m, 64);
+  return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
-// Outputs i0 .. i0 + count - 1 of merge(A[0..na), B[0..nb)), both
-// descending, into dst[i0 ..]: one
-// binary search for where output i0 splits A and B (merge path), then a
-// sequential walk, one comparison per output with the two heads in
-// registers.
-__device__ __forceinline__ void merge_run(const uint64_t* A, int na, const uint64_t* B, int nb, int i0, int count,
-                                          uint64_t* dst) {
-  int lo = i0 - nb > 0 ? i0 - nb : 0;
-  int hi = i0 < na ? i0 : na;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (A[mid] > B[i0 - mid - 1]) lo = mid + 1;
-    else hi = mid;
+// Largest and smallest nonzero of the block's keys (PER per thread).
+template <int PER>
+__device__ __forceinline__ void key_range(const uint64_t (&key)[PER], uint64_t& hi, uint64_t& lo, SelectLds& L) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  hi = 0;
+  lo = ~0ull;
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    hi = key[r] > hi ? key[r] : hi;
+    lo = key[r] != 0 && key[r] < lo ? key[r] : lo;
   }
-  int ia = lo, ib = i0 - lo;
-  uint64_t ha = ia < na ? A[ia] : 0, hb = ib < nb ? B[ib] : 0;
-  for (int k = 0; k < count; ++k) {
-    const bool take_a = ia < na && (ib >= nb || ha > hb);
-    if (take_a) {
-      dst[i0 + k] = ha;
-      ++ia;
-      ha = ia < na ? A[ia] : 0;
-    } else {
-      dst[i0 + k] = hb;
-      ++ib;
-      hb = ib < nb ? B[ib] : 0;
-    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t h = shfl_xor_u64(hi, o), l = shfl_xor_u64(lo, o);
+    hi = h > hi ? h : hi;
+    lo = l < lo ? l : lo;
+  }
+  if (lane == 0) {
+    L.hi[wave] = hi;
+    L.lo[wave] = lo;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    hi = L.hi[w] > hi ? L.hi[w] : hi;
+    lo = L.lo[w] < lo ? L.lo[w] : lo;
   }
 }
 
-constexpr int kRun = 8;  // outputs per thread per merge_run
+// Inclusive sum over the block's threads in order (one barrier).
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, SelectLds& L) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t o = __shfl_up(v, d, 64);
+    if (lane >= d) v += o;
+  }
+  if (lane == 63) L.wsum[wave] = v;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) v += w < wave ? L.wsum[w] : 0u;
+  return v;
+}
 
-// Merge `n` lists (list l at src + l * K, length len[l]) pairwise down to
-// one, ping-ponging between src and dst; returns the buffer holding it (at
-// offset 0) and its length in len[0].  All threads of the block call this.
-__device__ uint64_t* merge_tree(uint64_t* src, uint64_t* dst, int* len, int n, int K) {
-  while (n > 1) {
-    const int pairs = n >> 1;
-    const int runs = (K + kRun - 1) / kRun;  // per pair
-    for (int t = threadIdx.x; t < pairs * runs; t += blockDim.x) {
-      const int p = t / runs, i0 = (t - p * runs) * kRun;
-      const int la = len[2 * p], lb = len[2 * p + 1];
-      const int lim = la + lb < K ? la + lb : K;
-      if (i0 < lim)
-        merge_run(src + 2 * p * K, la, src + (2 * p + 1) * K, lb, i0, lim - i0 < kRun ? lim - i0 : kRun,
-                  dst + p * K);
-    }
-    // an odd list out is carried over unchanged
-    if (n & 1)
-      for (int i = threadIdx.x; i < len[n - 1]; i += blockDim.x) dst[pairs * K + i] = src[(n - 1) * K + i];
+// A threshold that at least K and at most `cap` >= K of the block's `n` keys
+// (PER per thread, 0: none; all distinct) reach; 1 when n <= cap.  1024
+// threads, all of which call this with the same n, K, cap.
+template <int PER>
+__device__ __forceinline__ uint64_t select_top(const uint64_t (&key)[PER], int n, int K, int cap, SelectLds& L) {
+  if (n <= cap) return 1;
+  uint64_t hi, lo;
+  key_range<PER>(key, hi, lo, L);
+  uint32_t sure = 0;  // keys above hi
+  for (;;) {
+    const uint64_t range = hi - lo;
+    const int bits = range == 0 ? 0 : 64 - __builtin_clzll(range);
+    const int shift = bits > 11 ? bits - 11 : 0;  // 2048 bins
+    L.hist[threadIdx.x] = L.hist[threadIdx.x + 1024] = 0;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int p = 0; p < pairs; ++p) {
-        const int s = len[2 * p] + len[2 * p + 1];
-        len[p] = s < K ? s : K;
+#pragma unroll
+    for (int r = 0; r < PER; ++r)
+      if (key[r] >= lo && key[r] <= hi) atomicAdd(&L.hist[(hi - key[r]) >> shift], 1u);
+    __syncthreads();
+    // bins 2 t and 2 t + 1 of thread t, scanned over the block
+    const uint32_t c0 = L.hist[2 * threadIdx.x], c1 = L.hist[2 * threadIdx.x + 1];
+    const uint32_t run = block_scan(c0 + c1, L);
+    const uint32_t need = static_cast<uint32_t>(K) - sure;
+    const uint32_t b0 = run - c0 - c1, b1 = run - c1;  // keys before each bin
+    if (b0 < need && need <= b1) {
+      L.edge[0] = 2 * threadIdx.x;
+      L.edge[1] = b0;
+      L.at = c0;
+    } else if (b1 < need && need <= run) {
+      L.edge[0] = 2 * threadIdx.x + 1;
+      L.edge[1] = b1;
+      L.at = c1;
+    }
+    __syncthreads();
+    const uint64_t bin = L.edge[0];
+    const uint32_t before = static_cast<uint32_t>(L.edge[1]), in = L.at;
+    const uint64_t top = hi - (bin << shift);  // the bin holds keys top - width + 1 .. top
+    const uint64_t width = 1ull << shift;
+    const uint64_t low = top - lo < width ? lo : top - width + 1;
+    if (sure + before + in <= static_cast<uint32_t>(cap) || shift == 0) return low;
+    sure += before;
+    hi = top;
+    lo = low;
+  }
+}
+
+// Position threadIdx.x + 1024 r of lists of K entries as (list, entry).
+struct ListAt {
+  int l, i, dl, di;
+  __device__ __forceinline__ explicit ListAt(int K)
+      : l(static_cast<int>(threadIdx.x) / K), i(static_cast<int>(threadIdx.x) % K), dl(1024 / K), di(1024 % K) {}
+  __device__ __forceinline__ void next(int K) {
+    l += dl;
+    i += di;
+    if (i >= K) {
+      i -= K;
+      ++l;
+    }
+  }
+};
+
+// Sorts the first `n` <= 1024 keys of `keys` descending in place: each key's
+// place is its bin's start (2048 bins over the keys' range) plus its rank
+// among the few keys of its bin.  Keys that crowd a bin (more than 32) are
+// sorted by a bitonic network instead.  `buf` holds 1024 keys; 1024 threads.
+__device__ __forceinline__ void sort_desc(uint64_t* keys, int n, uint64_t* buf, SelectLds& L) {
+  const int t = threadIdx.x;
+  const uint64_t key[1] = {t < n ? keys[t] : 0};
+  if (n <= 64) {  // one wave, in registers
+    if (t < 64) {
+      uint64_t v = key[0];
+#pragma unroll
+      for (int k = 2; k <= 64; k <<= 1)
+#pragma unroll
+        for (int j = k >> 1; j > 0; j >>= 1) {
+          const uint64_t o = shfl_xor_u64(v, j);
+          const bool want_max = ((t & j) == 0) == ((t & k) == 0);
+          v = want_max == (v < o) ? o : v;
+        }
+      keys[t] = v;
+    }
+    __syncthreads();
+    return;
+  }
+  uint64_t hi, lo;
+  key_range<1>(key, hi, lo, L);
+  const uint64_t range = n > 0 ? hi - lo : 0;
+  const int bits = range == 0 ? 0 : 64 - __builtin_clzll(range);
+  const int shift = bits > 11 ? bits - 11 : 0;
+  L.hist[t] = L.hist[t + 1024] = 0;
+  if (t == 0) L.at = 0;
+  __syncthreads();
+  const uint32_t bin = t < n ? static_cast<uint32_t>((hi - key[0]) >> shift) : 0u;
+  const uint32_t r = t < n ? atomicAdd(&L.hist[bin], 1u) : 0u;
+  __syncthreads();
+  const uint32_t c0 = L.hist[2 * t], c1 = L.hist[2 * t + 1];
+  if (c0 > 32 || c1 > 32) L.at = 1;
+  const uint32_t run = block_scan(c0 + c1, L);
+  L.hist[2 * t] = run - c0 - c1;
+  L.hist[2 * t + 1] = run - c1;
+  __syncthreads();
+  if (L.at == 0) {
+    uint32_t s = 0, e = 0;
+    if (t < n) {
+      s = L.hist[bin];
+      e = bin + 1 < kBins ? L.hist[bin + 1] : static_cast<uint32_t>(n);
+      buf[s + r] = key[0];
+    }
+    __syncthreads();
+    uint32_t place = s;
+    for (uint32_t m = s; m < e; ++m) place += buf[m] > key[0] ? 1u : 0u;
+    if (t < n) keys[place] = key[0];
+    __syncthreads();
+    return;
+  }
+  uint64_t v = key[0];
+  int width = 2;
+  while (width < n) width <<= 1;
+  for (int k = 2; k <= width; k <<= 1) {
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      uint64_t o;
+      if (j < 64) {
+        o = shfl_xor_u64(v, j);
+      } else {
+        __syncthreads();
+        buf[t] = v;
+        __syncthreads();
+        o = buf[t ^ j];
       }
-      if (n & 1) len[pairs] = len[n - 1];
+      const bool want_max = ((t & j) == 0) == ((t & k) == 0);
+      v = want_max == (v < o) ? o : v;
     }
-    __syncthreads();
-    uint64_t* t = src;
-    src = dst;
-    dst = t;
-    n = pairs + (n & 1);
   }
-  return src;
+  __syncthreads();
+  keys[t] = v;
+  __syncthreads();
 }
 
+constexpr int kRowBytes = 1024;   // widest allow row looked up through LDS
 constexpr int kSliceWaves = 16;  // one wave per beam of a slice (BS <= 16)
 
 __global__ __launch_bounds__(64 * kSliceWaves) void genrec_slice_topk(GenrecArgs a) {
-  __shared__ uint64_t bufA[kListKeys];
-  __shared__ uint64_t bufB[kListKeys];
-  __shared__ int len[64];
+  static_assert(kSliceWaves == 16, "select_top's 1024 threads");
+  __shared__ uint64_t buf[kListKeys];
+  __shared__ SelectLds sel;
+  __shared__ __attribute__((aligned(16))) uint8_t rows[kSliceWaves][kRowBytes];  // the beams' rows of the allow table
+  __shared__ int len[kSliceWaves];
+  __shared__ uint32_t cursor;
   const int n = blockIdx.x / a.S, s = blockIdx.x - (blockIdx.x / a.S) * a.S;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b0 = s * a.BS;
   const int nb = a.BW - b0 < a.BS ? a.BW - b0 : a.BS;
   const bool mask = a.apply_mask && a.allow != nullptr && a.nodes != nullptr;
-  // each wave compacts beams wave, wave + kSliceWaves, ... (one each when
-  // BS <= kSliceWaves): list of beam j at bufA + j * K.
-  // A beam's candidates go in groups of kPre chunks of 64: the scores and
-  // tokens of the whole group are loaded, then all of its trie lookups are
-  // issued, then the chunks are compacted in order (ballot prefix sums,
-  // stopping at K): two memory round trips per group instead of two per
-  // chunk.  Which candidates are taken, and where, is unchanged.
+  // wave j compacts beam j of the slice (BS <= kSliceWaves): its list at
+  // buf + j * K.  The beam's candidates go in groups of kPre chunks of 64: the
+  // scores and tokens of the whole group are loaded, then all of its trie
+  // lookups are issued, then the chunks are compacted in order (ballot prefix
+  // sums, stopping at K): two memory round trips per group.  Loads are
+  // unconditional on clamped indices: under a lane's condition each would
+  // wait for the one before it.
   constexpr int kPre = 16;
-  for (int j = wave; j < nb; j += kSliceWaves) {
-    const int b = b0 + j;
+  if (wave < nb) {
+    const int b = b0 + wave;
     const float cb = a.cum[static_cast<int64_t>(n) * a.BW + b];
     const int64_t node = mask ? a.nodes[static_cast<int64_t>(n) * a.BW + b] : -1;
     const float* lpb = a.lp + (static_cast<int64_t>(n) * a.BW + b) * a.C;
     const int64_t* tkb = a.tok + (static_cast<int64_t>(n) * a.BW + b) * a.C;
+    const bool lookup = node >= 0 && a.n_nodes > 0 && a.vsz > 0;  // (node < 0 accepts every token)
+    const uint8_t* allow = nullptr;
+    if (lookup) allow = a.allow + (node > a.n_nodes - 1 ? a.n_nodes - 1 : node) * a.vsz;
+    // A row of up to 1 KB is read once, 16 bytes a lane, and looked up in LDS:
+    // 1024 candidates are 16 gathers of 64 single bytes, and a gather takes
+    // the address path a cycle a lane (8 us of a 512-beam step).
+    const bool staged = lookup && a.vsz <= kRowBytes && a.vsz % 16 == 0 && (reinterpret_cast<uintptr_t>(allow) & 15) == 0;
+    if (staged && 16 * lane < a.vsz)
+      *reinterpret_cast<u32x4*>(rows[wave] + 16 * lane) = *reinterpret_cast<const u32x4*>(allow + 16 * lane);
     int count = 0;
     for (int g0 = 0; g0 < a.C && count < a.K; g0 += 64 * kPre) {
       float v[kPre];
-      int64_t tk[kPre];
+      int64_t rel[kPre];
 #pragma unroll
       for (int u = 0; u < kPre; ++u) {
-        const int c = g0 + 64 * u + lane;
-        v[u] = c < a.C ? cb + lpb[c] : 0.0f;
-        tk[u] = c < a.C && mask ? tkb[c] : 0;
+        const int c = g0 + 64 * u + lane, cc = c < a.C ? c : a.C - 1;
+        v[u] = cb + lpb[cc];
+        rel[u] = lookup ? tkb[cc] - a.token_base : 0;
       }
-      bool okv[kPre];
+      uint32_t in[kPre] = {};
+      if (staged) {
 #pragma unroll
-      for (int u = 0; u < kPre; ++u) {
-        const int c = g0 + 64 * u + lane;
-        bool ok = c < a.C && v[u] == v[u];  // NaN: never picked
-        if (mask) ok = ok && v[u] != a.neg_inf && cand_ok(a, node, tk[u]);
-        okv[u] = ok;
+        for (int u = 0; u < kPre; ++u) in[u] = rows[wave][rel[u] >= 0 && rel[u] < a.vsz ? rel[u] : 0];
+      } else if (lookup) {
+#pragma unroll
+        for (int u = 0; u < kPre; ++u) in[u] = allow[rel[u] >= 0 && rel[u] < a.vsz ? rel[u] : 0];
       }
 #pragma unroll
       for (int u = 0; u < kPre; ++u) {
-        if (count >= a.K) break;
         const int c = g0 + 64 * u + lane;
-        const uint64_t bal = __ballot(okv[u]);
+        bool ok = c < a.C && count < a.K && v[u] == v[u];  // NaN: never picked
+        if (mask) ok = ok && v[u] != a.neg_inf && (node < 0 || lookup);
+        if (lookup) ok = ok && rel[u] >= 0 && rel[u] < a.vsz && in[u] != 0;
+        const uint64_t bal = __ballot(ok);
         const int pos = count + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
                                     static_cast<uint32_t>(bal >> 32),
                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal), 0u)));
-        if (okv[u] && pos < a.K) bufA[j * a.K + pos] = make_key(v[u], static_cast<uint32_t>(b * a.C + c));
+        if (ok && pos < a.K) buf[wave * a.K + pos] = make_key(v[u], static_cast<uint32_t>(b * a.C + c));
         count += __builtin_popcountll(bal);
       }
     }
-    if (lane == 0) len[j] = count < a.K ? count : a.K;
+    if (lane == 0) len[wave] = count < a.K ? count : a.K;
+  } else if (lane == 0) {
+    len[wave] = 0;
   }
+  if (threadIdx.x == 0) cursor = 0;
   __syncthreads();
-  uint64_t* res = merge_tree(bufA, bufB, len, nb, a.K);
-  uint64_t* out = a.scratch + (static_cast<int64_t>(n) * a.S + s) * (1 + a.K);
-  for (int i = threadIdx.x; i < len[0]; i += blockDim.x) out[1 + i] = res[i];
-  if (threadIdx.x == 0) out[0] = static_cast<uint64_t>(len[0]);
+  int total = 0;
+#pragma unroll
+  for (int j = 0; j < kSliceWaves; ++j) total += len[j];
+  uint64_t* const out = a.scratch + (static_cast<int64_t>(n) * a.S + s) * (1 + a.K);
+  if (threadIdx.x == 0) out[0] = static_cast<uint64_t>(total < a.K ? total : a.K);
+  constexpr int kPer = kListKeys / 1024;
+  uint64_t key[kPer];
+  ListAt at(a.K);
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const bool ok = at.l < nb && at.i < len[at.l < nb ? at.l : 0];
+    key[r] = ok ? buf[threadIdx.x + r * 1024] : 0;
+    at.next(a.K);
+  }
+  // the rest of the list: 0, no key (kernel 2 then reads whole lists without
+  // waiting for their lengths)
+  for (int i = total + static_cast<int>(threadIdx.x); i < a.K; i += 1024) out[1 + i] = 0;
+  const uint64_t least = select_top<kPer>(key, total, a.K, a.K, sel);
+#pragma unroll
+  for (int r = 0; r < kPer; ++r)
+    if (key[r] >= least) out[1 + atomicAdd(&cursor, 1u)] = key[r];
 }
 
 __global__ __launch_bounds__(1024) void genrec_request_topk_expand(GenrecArgs a) {
-  __shared__ uint64_t bufA[kListKeys];
-  __shared__ uint64_t bufB[kListKeys];
-  __shared__ uint64_t acc[1024];  // running top K of the groups merged so far
+  __shared__ uint64_t acc[1024];  // keys that hold the top K of the lists read so far
+  __shared__ SelectLds sel;
   __shared__ int len[64];
-  __shared__ int acc_len;
+  __shared__ uint32_t cursor;
   __shared__ int64_t sel_parent[1024];
   __shared__ int64_t sel_token[1024];
   const int n = blockIdx.x;
   const int K = a.K;
   const uint64_t* lists = a.scratch + static_cast<int64_t>(n) * a.S * (1 + K);
-  // The slice lists go in groups of G that fill an LDS buffer: a group is
-  // copied in (coalesced, one memory round trip), merged down to one list
-  // in LDS and folded into acc.  (Merging straight from the scratch would
-  // put a dependent global read at every step of every binary search.)
-  const int G = kListKeys / K < 64 ? kListKeys / K : 64;  // (len[] holds 64)
-  if (threadIdx.x == 0) acc_len = 0;
+  // The slices' lists go in groups of G that fill the threads' registers; the
+  // keys kept from the groups before ride along.
+  constexpr int kPer = 16;
+  const int G = kPer * 1024 / K < 64 ? kPer * 1024 / K : 64;  // (len[] holds 64)
+  // keys kept: up to twice K's power of two, so that one histogram pass mostly
+  // does and the sort below stays short
+  int cap = 2;
+  while (cap < K) cap <<= 1;
+  cap = cap < 512 ? 2 * cap : 1024;
+  int held = 0;
   for (int g0 = 0; g0 < a.S; g0 += G) {
     const int gs = a.S - g0 < G ? a.S - g0 : G;
     const uint64_t* gl = lists + static_cast<int64_t>(g0) * (1 + K);
-    if (threadIdx.x < gs) len[threadIdx.x] = static_cast<int>(gl[static_cast<int64_t>(threadIdx.x) * (1 + K)]);
-    __syncthreads();
-    // the keys of every list of the group (gs * K <= kListKeys = 8 per
-    // thread of 1024): all loads issued before any is stored
-    constexpr int kPer = kListKeys / 1024;
-    uint64_t key[kPer];
+    if (threadIdx.x == 0) cursor = 0;
+    uint64_t key[kPer + 1];
+    ListAt at(K);
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-      const int t = threadIdx.x + r * 1024;
-      const int l = t / K, i = t - l * K;
-      key[r] = (l < gs && i < len[l]) ? gl[static_cast<int64_t>(l) * (1 + K) + 1 + i] : 0;
+      const uint64_t x = gl[at.l < gs ? static_cast<uint32_t>(at.l * (1 + K) + 1 + at.i) : 0u];
+      key[r] = at.l < gs ? x : 0;
+      at.next(K);
     }
+    if (threadIdx.x < 64)
+      len[threadIdx.x] = static_cast<int>(threadIdx.x) < gs ? static_cast<int>(gl[threadIdx.x * (1 + K)]) : 0;
+    __syncthreads();
+    key[kPer] = static_cast<int>(threadIdx.x) < held ? acc[threadIdx.x] : 0;
+    int total = len[threadIdx.x & 63];
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int t = threadIdx.x + r * 1024;
-      const int l = t / K, i = t - l * K;
-      if (l < gs && i < len[l]) bufA[l * K + i] = key[r];
-    }
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+    total += held;
+    __syncthreads();  // acc, len and the cursor are read
+    const uint64_t least = select_top<kPer + 1>(key, total, K, cap, sel);
+#pragma unroll
+    for (int r = 0; r <= kPer; ++r)
+      if (key[r] != 0 && key[r] >= least) acc[atomicAdd(&cursor, 1u)] = key[r];
     __syncthreads();
-    uint64_t* res = merge_tree(bufA, bufB, len, gs, K);
-    uint64_t* other = res == bufA ? bufB : bufA;
-    const int lr = len[0], la = acc_len;
-    const int lt = la + lr < K ? la + lr : K;
-    for (int i0 = threadIdx.x * kRun; i0 < lt; i0 += blockDim.x * kRun)
-      merge_run(acc, la, res, lr, i0, lt - i0 < kRun ? lt - i0 : kRun, other);
-    __syncthreads();
-    for (int i = threadIdx.x; i < lt; i += blockDim.x) acc[i] = other[i];
-    if (threadIdx.x == 0) acc_len = lt;
+    held = static_cast<int>(cursor);
     __syncthreads();
   }
+  sort_desc(acc, held, reinterpret_cast<uint64_t*>(sel_parent), sel);
   const uint64_t* res = acc;
-  const int got = acc_len;
+  const int got = held < K ? held : K;
   const int64_t* tkn = a.tok + static_cast<int64_t>(n) * a.BW * a.C;
   for (int k = threadIdx.x; k < K; k += blockDim.x) {
     float v = a.neg_inf;
