@@ -4,7 +4,7 @@
 // python/flashrec/engine/graph.py:33-43 and :186-193).
 //
 // One 256-thread workgroup per row.  The row is read once into registers as
-// 48-bit composite keys (order-preserving score bits << 16 | (0xFFFF - index))
+// composite keys (order-preserving score bits << 32 | (0xFFFF - index))
 // so that every key is distinct and equal scores rank by ascending index.
 // A coarse pass bins the keys into 2048 ranges spanning the row's finite key
 // (or score) range (LDS histogram + block scan): keys in bins above the C-th
@@ -47,7 +47,7 @@ __device__ __forceinline__ uint32_t score_bits(float v) {
 }
 
 __device__ __forceinline__ uint64_t comp_key(uint32_t bits, uint32_t idx) {
-  return (static_cast<uint64_t>(bits) << 16) | static_cast<uint64_t>(0xFFFFu - idx);
+  return (static_cast<uint64_t>(bits) << 32) | static_cast<uint64_t>(0xFFFFu - idx);
 }
 
 // score_bits of a finite value.
@@ -118,8 +118,8 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
   __shared__ uint32_t wsum[kThreads / 64];
   __shared__ uint32_t red[3 * (kThreads / 64)];
   __shared__ uint32_t sel[4];
-  __shared__ uint64_t sk[N];
-  __shared__ uint64_t cl[64];
+  __shared__ uint64_t sk[N + 64];  // the taken keys, then the boundary bin's candidates
+  uint64_t* const cl = sk + N;
   __shared__ float lred[8];
 
   const int t = threadIdx.x;
@@ -143,6 +143,14 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
   // 84.5 -> 80.4 (by score: 91.2), logits 167 -> 78.  Other rows (masked
   // entries of -1e9 or the lowest float, infinities, NaNs) keep the clamped
   // bins over the key's bits.
+  // Then, 80.4 -> 74.7 and 78 -> 67.7 (50 rows, top 100: 10.8 -> 9.5 and 9.2 ->
+  // 7.9): the key's index in a word of its own, one store per taken key
+  // whichever part it goes to, and one branch, not one per key, on the form of
+  // the row.  134 MB in and 50 MB out are 36 us of copying; of the 80.0 before,
+  // loading with the log-softmax took 28.2, the histogram 3.7, its scan 7.1,
+  // the compaction 14.7, the order inside the bins and the stores 26.3.  Five
+  // waves per SIMD instead of four spill (logits 67.7 -> 84.7); ranking a
+  // thread's keys together and storing along the row was 2 us slower.
   uint32_t key[NK];
   float lse = 0.0f;
   constexpr bool LIN = FULL && !LSM;  // quick rows are binned by score
@@ -191,10 +199,13 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
       kmax = kfmax = uni(finite_bits(vmx));
       kfmin = uni(finite_bits(vmn));
     }
+    // (one branch around each loop: inside, it would be taken per key)
+    if (quick) {
 #pragma unroll
-    for (int q = 0; q < NK; ++q) {
-      const float y = v[q >> 2][q & 3];
-      key[q] = !quick ? score_bits(y) : LIN ? __float_as_uint(y) : finite_bits(y);
+      for (int q = 0; q < NK; ++q) key[q] = LIN ? __float_as_uint(v[q >> 2][q & 3]) : finite_bits(v[q >> 2][q & 3]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NK; ++q) key[q] = score_bits(v[q >> 2][q & 3]);
     }
     __syncthreads();  // (red is written again below)
   } else {
@@ -315,7 +326,8 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
         sel[2] = c[i];
         sel[3] = run;      // keys surely taken
       }
-      hist[t * BPT + i] = run;  // bin start; a cursor below
+      // the cursor of the compaction: bin start, for bin b* the candidates'
+      hist[t * BPT + i] = run < C && C <= run + c[i] ? N : run;
       run += c[i];
     }
   }
@@ -341,7 +353,7 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
   const bool bin_sort = uni(lmax) <= kSegMax && cntb <= 64;
 
   // ---- compaction: sure keys into their bin's range of the sort buffer;
-  // candidates of bin b* into a short list when they fit one wave (else the
+  // candidates of bin b* into a short list behind it when they fit one wave (else the
   // exact radix pass below resolves them)
   const bool short_list = cntb <= 64;
   // slots are claimed eight keys at a time so the atomics' round trips overlap
@@ -363,8 +375,7 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
 #pragma unroll
       for (int u = 0; u < SB; ++u) {
         const int q = q0 + u;
-        if (slot[u] < sure) sk[slot[u]] = comp_key(bits(q), index_of(q));
-        else if (slot[u] != 0xFFFFFFFFu) cl[slot[u] - sure] = comp_key(bits(q), index_of(q));
+        if (slot[u] != 0xFFFFFFFFu) sk[slot[u]] = comp_key(bits(q), index_of(q));
       }
     }
   };
@@ -398,7 +409,7 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
 #pragma unroll
       for (int q = 0; q < NK; ++q) {
         if (valid(q) && bin_key(key[q]) == bstar) {
-          const uint32_t d = kmax - key[q];
+          const uint32_t d = fresh_s(kmax) - key[q];
           const uint32_t idx = index_of(q);
           bool match;
           uint32_t digit;
@@ -444,7 +455,7 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
     uint32_t mine = 0;
     auto admitted = [&](int q) -> bool {
       if (!valid(q) || bin_key(key[q]) != bstar) return false;
-      const uint32_t d = kmax - key[q];
+      const uint32_t d = fresh_s(kmax) - key[q];
       if (!ip) return (d >> sh) <= P;
       return d < D || (d == D && (index_of(q) >> ish) <= Pi);
     };
@@ -463,7 +474,7 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
     const int64_t idx = 0xFFFF - static_cast<int64_t>(kk & 0xFFFFu);
     // the score from its key; zeros (either sign) and NaNs are re-read so
     // that their bits come out as stored
-    const uint32_t kb = static_cast<uint32_t>(kk >> 16);
+    const uint32_t kb = static_cast<uint32_t>(kk >> 32);
     const float val = (kb == 0x80000000u || kb == 0xFFFFFFFFu)
                           ? (LSM ? xr[idx] - lse : xr[idx])
                           : __uint_as_float((kb & 0x80000000u) ? (kb & 0x7FFFFFFFu) : ~kb);
@@ -479,7 +490,7 @@ __global__ __launch_bounds__(kThreads) void row_topk_kernel(TopkArgs a) {
       const uint64_t kk = sk[i];
       int f = i;
       if (static_cast<uint32_t>(i) < sure) {
-        const uint32_t b = bin_key(static_cast<uint32_t>(kk >> 16));
+        const uint32_t b = bin_key(static_cast<uint32_t>(kk >> 32));
         const uint32_t s = b == 0 ? 0u : hist[b - 1], e = hist[b];
         uint32_t r = 0;
         for (uint32_t m = s; m < e; ++m) r += sk[m] > kk ? 1u : 0u;
