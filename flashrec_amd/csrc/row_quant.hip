@@ -6,7 +6,8 @@
 // stride.  The row is read once with 16-byte loads (8 bf16 per lane per
 // vector), kept in VGPRs, reduced with cross-lane shuffles (no LDS, no
 // barriers), and written once with coalesced 8-byte (e4m3) or 16-byte (bf16)
-// stores.  Rows wider than the register budget, or with unaligned
+// stores.  Aligned fp16 and fp32 rows take row_kernel_fine, a workgroup per
+// row read once.  Rows wider than the register budget, or with unaligned
 // widths/strides, take a generic three-pass kernel with the same arithmetic.
 //
 // These kernels issue more VALU work per byte than the HBM can deliver
@@ -69,8 +70,8 @@ __device__ __forceinline__ void unpack8(const u32x4& v, float* f) {
 // SiLU of bf16 rows: the same arithmetic as the vector kernel and the GEMM's
 // SiLU epilogue (silu_in_range for |g| <= 80, torch's formula beyond), so a
 // bf16 row gives the same bits whichever kernel takes it (aligned or not,
-// GEMM epilogue or row kernel).  fp16 and fp32 rows only ever take this
-// kernel and keep torch's formula: their finer roundings (fp16 subnormals,
+// GEMM epilogue or row kernel).  fp16 and fp32 rows keep torch's formula in
+// both kernels that take them: their finer roundings (fp16 subnormals,
 // unrounded fp32) show the last-ulp differences of the in-range form.
 template <int DT>
 __device__ __forceinline__ float silu_any(float g) {
