@@ -13,6 +13,7 @@ only its output and can be captured.
 
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Dict, List, Optional, Tuple
 
 import torch
@@ -68,8 +69,9 @@ class AttentionBackend:
                 "indices": torch.zeros(bs * max_seq_len, dtype=torch.int32, device=dev),
                 "last": torch.ones(bs, dtype=torch.int32, device=dev),
                 "kv_len": torch.zeros(bs, dtype=torch.int32, device=dev),
-                "group_prefix": torch.zeros(max(plan_size(bs, self.num_qo_heads, self.num_kv_heads), 1),
-                                            dtype=torch.int32, device=dev),
+                "group_prefix": _plan_rows(
+                    torch.zeros(plan_size(bs, self.num_qo_heads, self.num_kv_heads), dtype=torch.int32, device=dev),
+                    bs, self.num_qo_heads, self.num_kv_heads),
             }
 
     def graph_bufs(self, bs: int) -> Optional[dict]:
@@ -99,7 +101,7 @@ class AttentionBackend:
         bufs = self._graph_bufs.get(self._graph_bs) if self._graph_bs is not None else None
         gp = None
         if bufs is not None and not batch.is_prefill:
-            gp = bufs["group_prefix"][: max(plan_size(n, self.num_qo_heads, self.num_kv_heads), 1)]
+            gp = bufs["group_prefix"]
         self._plan["group_prefix"] = attention_plan(self._plan["indices"], self._plan["start"],
                                                     self._plan["len"], self.num_qo_heads,
                                                     self.num_kv_heads, out=gp)
@@ -176,43 +178,88 @@ class AttentionBackend:
 
 
 def plan_size(T: int, hq: int, hk: int) -> int:
-    """Entries of an attention plan for T query tokens: one per group of 32 /
-    (hq / hk) of them, then two per token."""
+    """Entries of an attention plan's buffer for T query tokens: one record per
+    group of 32 / (hq / hk) of them."""
     n = int(load().fr_paged_attention_plan_size(int(T), int(hq), int(hk)))
     if n < 0:
         raise ValueError(f"unsupported head ratio {hq}/{hk}")
     return n
 
 
+@lru_cache(maxsize=64)
+def _record_size(hq: int, hk: int) -> int:
+    return plan_size(1, hq, hk)
+
+
+def _groups(T: int, hq: int, hk: int) -> Tuple[int, int]:
+    """(query groups of T tokens, entries of a group's record)."""
+    stride = _record_size(int(hq), int(hk))
+    return -(-int(T) * (int(hq) // int(hk)) // 32), stride
+
+
+def _plan_rows(buf: torch.Tensor, T: int, hq: int, hk: int) -> torch.Tensor:
+    """The records at the front of a flat plan buffer as attention_plan returns
+    them: a strided view with one entry, its shared prefix, per group."""
+    groups, stride = _groups(T, hq, hk)
+    return buf.reshape(-1)[: groups * stride].view(groups, stride)[:, 0]
+
+
+def _plan_records(plan: torch.Tensor, groups: int, stride: int) -> bool:
+    """Whether ``plan`` (a view as _plan_rows makes it, or a flat buffer) has
+    room for the whole records of ``groups`` groups."""
+    if plan.dim() == 1 and plan.numel() >= groups and plan.stride(0) == stride:
+        return plan.storage_offset() + groups * stride <= plan.untyped_storage().nbytes() // 4
+    return plan.is_contiguous() and plan.numel() >= groups * stride
+
+
+def _check_plan_buffer(plan: torch.Tensor, groups: int, records: bool) -> None:
+    if plan.dtype != torch.int32 or not (records or plan.is_contiguous()) or plan.numel() < groups:
+        raise ValueError(f"a plan is what attention_plan returns for the same slot lists, at least {groups} groups "
+                         "of them, or a contiguous int32 tensor of as many entries")
+    require_device(plan)
+
+
 def attention_plan(kv_indices: torch.Tensor, kv_start: torch.Tensor, kv_len: torch.Tensor,
                    hq: int, hk: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The shared slot prefix (rounded down to 32) of each group of 32 / (hq /
-    hk) consecutive query tokens, then the kernels' own entries (how a group's
-    tokens fall into runs with common keys): computed once per batch, passed
-    to every layer's ``paged_attention`` as ``group_prefix``."""
+    hk) consecutive query tokens: computed once per batch, passed to every
+    layer's ``paged_attention`` as ``group_prefix``.  What is returned is a
+    strided view of one record per group, which holds the kernels' own entries
+    too (how the group's tokens fall into runs with common keys); ``out`` may
+    be such a view, a flat buffer of ``plan_size`` entries, which it then views,
+    or a contiguous tensor of one entry per group, which receives the prefixes
+    alone."""
     require_device(kv_indices, kv_start, kv_len)
     T = int(kv_start.numel())
-    n = plan_size(T, hq, hk)
-    if out is None:
-        out = torch.empty(max(n, 1), dtype=torch.int32, device=kv_start.device)
-    if out.dtype != torch.int32 or not out.is_contiguous() or out.numel() < n:
-        raise ValueError("plan buffer must be contiguous int32 with plan_size entries")
+    groups, stride = _groups(T, hq, hk)
+    plan = out
+    if out is None or not _plan_records(out, groups, stride):
+        if out is not None:
+            _check_plan_buffer(out, groups, False)
+        plan = torch.empty(max(groups, 1) * stride, dtype=torch.int32, device=kv_start.device)
+    else:
+        _check_plan_buffer(out, groups, True)
     call("fr_paged_attention_plan", kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
-         T, int(hq), int(hk), out.data_ptr(), stream_of(kv_start))
-    return out
+         T, int(hq), int(hk), plan.data_ptr(), stream_of(kv_start))
+    if plan is out and out.stride(-1) == stride:
+        return out
+    rows = _plan_rows(plan, T, hq, hk)
+    if out is not None and plan is not out:
+        out.view(-1)[:groups].copy_(rows)
+        return out
+    return rows
 
 
 def _check_plan(group_prefix: Optional[torch.Tensor], T: int, hq: int, hk: int) -> int:
-    """The plan's device pointer (0 for none) after checking it holds the
-    entries the kernels read for T tokens."""
+    """The device pointer of the plan's records after checking that it holds
+    those the kernels read for T tokens; 0, and each call finds the shared
+    prefixes itself, without a plan and for one of bare prefixes."""
     if group_prefix is None:
         return 0
-    n = plan_size(T, hq, hk)
-    if group_prefix.dtype != torch.int32 or not group_prefix.is_contiguous() or group_prefix.numel() < n:
-        raise ValueError(f"group_prefix must be a contiguous int32 plan of at least {n} entries "
-                         "(attention_plan over the same slot lists)")
-    require_device(group_prefix)
-    return group_prefix.data_ptr()
+    groups, stride = _groups(T, hq, hk)
+    records = _plan_records(group_prefix, groups, stride)
+    _check_plan_buffer(group_prefix, groups, records)
+    return group_prefix.data_ptr() if records else 0
 
 
 def _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len):

@@ -25,6 +25,7 @@
 // bits).  Output bf16.
 #include <type_traits>
 
+#include "attn_plan.h"
 #include "fr_common.h"
 
 namespace fr {
@@ -43,7 +44,7 @@ struct AttnArgs {
   int64_t T, Hq, Hk, num_slots;
   uint32_t row16;  // slot stride of both caches in 16-byte units, 0 where they differ or offsets pass 2^32
   float qscale;  // softmax scale * log2(e)
-  const int32_t* gp;  // the plan (attn_group_plan), or null
+  const int32_t* gp;  // the plan (attn_plan.h), or null
 };
 
 // Longest slot prefix shared by the `count` tokens from t0 on (count <= TOK).
@@ -224,8 +225,9 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, uint8_t* stage
   // Blocks of 32 key rows.  Block b < nshared: row r is position 32 b + r of
   // the common list; after that, row r holds position shared + (b - nshared) *
   // NREP + r % NREP of token r / NREP's own list, and each query only sees its
-  // own token's rows.
-  const int32_t P = seg.one_list ? maxlen : seg.shared;
+  // own token's rows.  (No more common positions than the shortest list has,
+  // whatever a plan made for other lists says.)
+  const int32_t P = seg.one_list ? maxlen : max(min(seg.shared, minlen), 0);
   const int32_t rest = seg.one_list ? 0 : maxlen - P;
   const int32_t nshared = (P + 31) / 32;
   const int32_t nblocks = nshared + (rest > 0 ? (rest + NREP - 1) / NREP : 0);
@@ -461,11 +463,8 @@ __device__ __forceinline__ Segment next_segment(const AttnArgs& a, int64_t t0, i
   return s;
 }
 
-// The plan, one wave per group, made once for every layer of a batch (entries
-// in fr_paged_attention_plan_size's order): the group's shared prefix rounded
-// down to 32; then for every token that starts a segment the number of its
-// tokens, negative where they read one list (0: the token continues one);
-// then the segments' shared prefixes.
+// The plan, one wave per group, made once for every layer of a batch (record
+// layout in attn_plan.h).
 template <int TOK>
 __global__ __launch_bounds__(256) void attn_group_plan(AttnArgs a, int32_t* gp, int64_t groups) {
   const int lane = threadIdx.x & 63;
@@ -474,62 +473,71 @@ __global__ __launch_bounds__(256) void attn_group_plan(AttnArgs a, int32_t* gp, 
   const int64_t t0 = group * TOK;
   const int ntok = static_cast<int>(min<int64_t>(TOK, a.T - t0));
   const bool ok = lane < ntok;
-  const int32_t start = a.kv_start[ok ? t0 + lane : t0], len = a.kv_len[ok ? t0 + lane : t0];
+  const int32_t start = a.kv_start[ok ? t0 + lane : t0];
   const int32_t p = tokens_prefix<TOK>(a, t0, ntok, lane);
-  if (lane == 0) gp[group] = p & ~31;
-  int32_t cnt = 0, sh = 0;  // lane tt: token t0 + tt's entries
+  int32_t cnt = 0, sh = 0;  // lane i: token t0 + i's entries
   if (p >= 32) {
-    const int32_t st = __builtin_amdgcn_readfirstlane(start);
-    const bool one = __ballot(ok && start != st) == 0;
-    cnt = lane == 0 ? (one ? -ntok : ntok) : 0;
+    cnt = lane == 0 ? ntok : 0;
     sh = lane == 0 ? p : 0;
   } else {
     const uint32_t linked = linked_tokens<TOK>(a, t0, ntok, lane);
     for (int at = 0; at < ntok;) {
       const Segment s = next_segment<TOK>(a, t0, ntok, linked, at, ok ? lane : TOK, start, 1, lane);
       if (lane == at) {
-        cnt = s.one_list ? -s.count : s.count;
+        cnt = s.count;
         sh = s.shared;
       }
       at += s.count;
     }
   }
-  if (ok) {
-    gp[groups + t0 + lane] = cnt;
-    gp[groups + a.T + t0 + lane] = sh;
+  int32_t* const rec = gp + group * plan_stride(TOK);
+  if (lane == 0) {
+    rec[0] = p & ~31;
+    rec[kPlanTag] = plan_tag(group);
+  }
+  if (lane < TOK) {
+    rec[kPlanCount + lane] = cnt;
+    rec[plan_shared_at(TOK) + lane] = sh;
   }
 }
 
-// A group's segments: from the plan, or found here.
+// A group's segments: from the plan's record, or found here (no plan, or a
+// buffer that holds no record of this group).
 template <int NREP>
 struct Segments {
   static constexpr int TOK = 32 / NREP;
   int64_t t0;
   int ntok;
   int32_t whole;  // prefix shared by the whole group rounded down to 32 (0: several segments)
-  int32_t cnt = 0, sh = 0;  // lane tt: the plan's entries of token t0 + tt
+  bool planned = false;
+  int32_t cnt = 0, sh = 0;  // lane i: the record's entries of token i
   uint32_t linked = 0;
   __device__ __forceinline__ Segments(const AttnArgs& a, int64_t t0_, int64_t group, int lane)
       : t0(t0_), ntok(static_cast<int>(min<int64_t>(TOK, a.T - t0_))) {
     if (a.gp) {
-      const int64_t groups = (a.T + TOK - 1) / TOK;
-      const int32_t* const e = a.gp + groups + t0 + (lane < ntok ? lane : 0);
-      whole = a.gp[group];
-      cnt = e[0];
-      sh = e[a.T];
-    } else {
+      const int32_t* const rec = a.gp + group * plan_stride(TOK);
+      const int i = lane < TOK ? lane : 0;
+      whole = rec[0];
+      cnt = rec[kPlanCount + i];
+      sh = rec[plan_shared_at(TOK) + i];
+      planned = __builtin_amdgcn_readfirstlane(rec[kPlanTag]) == plan_tag(group);
+    }
+    if (!planned) {
       whole = tokens_prefix<TOK>(a, t0, ntok, lane) & ~31;
       if (whole == 0) linked = linked_tokens<TOK>(a, t0, ntok, lane);
     }
   }
   __device__ __forceinline__ Segment at(const AttnArgs& a, int first, const Query& Q, bool single, int lane) const {
     if (single) return Segment{first, 1, 0, true};
-    if (a.gp) {
-      const int32_t c = __builtin_amdgcn_readlane(cnt, first);
-      return Segment{first, c < 0 ? -c : c, __builtin_amdgcn_readlane(sh, first), c < 0};
+    const int tok = (lane & 31) / NREP;
+    if (planned) {
+      const int count = plan_count(__builtin_amdgcn_readlane(cnt, first), first, ntok);
+      const int32_t st = __builtin_amdgcn_readlane(Q.start, first * NREP);
+      const bool one = __ballot(tok >= first && tok < first + count && Q.start != st) == 0;
+      return Segment{first, count, __builtin_amdgcn_readlane(sh, first), one};
     }
     if (whole > 0) return whole_group<TOK>(a, whole, Q.start, Q.len, Q.ok, NREP, lane);
-    return next_segment<TOK>(a, t0, ntok, linked, first, (lane & 31) / NREP, Q.start, NREP, lane);
+    return next_segment<TOK>(a, t0, ntok, linked, first, tok, Q.start, NREP, lane);
   }
 };
 
@@ -671,7 +679,7 @@ __global__ __launch_bounds__(64 * NW, 2) void paged_attn_split_d128(AttnArgs a) 
   if (segs.whole > 0) {
     const Segment s = segs.at(a, 0, Q, false, lane);
     attend_segment<NREP, false>(a, stage, kh, lane, Q, s, wave, NW, X, nan);
-    merge(s, X);
+    merge(Segment{0, 32 / NREP, 0, false}, X);  // tokens that the plan did not know: zeros
     return;
   }
   int single_until = 0;
@@ -928,7 +936,7 @@ static int64_t attn_groups(int64_t T, int64_t Hq, int64_t Hk) {
 
 extern "C" int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t Hk) {
   const int64_t groups = attn_groups(T, Hq, Hk);
-  return groups < 0 ? -1 : groups + 2 * T;
+  return groups < 0 ? -1 : groups * plan_stride(static_cast<int>(32 / (Hq / Hk)));
 }
 
 extern "C" int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries) {

@@ -275,15 +275,19 @@ int fr_paged_attention_split_fp8(const void* q, int64_t sqt, int64_t sqh, const 
 int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries);
 
 /* The per-batch attention plan, computed once for all layers that attend
- * over the same kv_indices / kv_start / kv_len: for each group of 32 / (Hq /
- * Hk) consecutive query tokens, the slot prefix all of them share, rounded
- * down to 32 (0: none); after these, for the attention kernels, how each
- * group's tokens fall into runs with common keys.  fr_paged_attention_plan_size
- * gives the entry count
- * (-1 for an unsupported head ratio).  Passing the plan as group_prefix to
- * fr_paged_attention_fp8 skips that detection in every call (null: each call
- * detects it).  No counterpart in the reference: flashinfer plans its own
- * decode batches (python/flashrec/attention/flashinfer.py:262-349). */
+ * over the same kv_indices / kv_start / kv_len: one record of fixed size per
+ * group of 32 / (Hq / Hk) consecutive query tokens.  A record's first entry is
+ * the slot prefix all of the group's tokens share, rounded down to 32 (0:
+ * none); the rest is the attention kernels' own (how the tokens fall into
+ * runs with common keys).  fr_paged_attention_plan_size gives the entries of
+ * the whole plan (int32; -1 for an unsupported head ratio).  Passing the plan
+ * as group_prefix to fr_paged_attention_fp8 skips that detection in every call
+ * (null: each call detects it).  A plan may be read by a call with fewer tokens
+ * than it was made for; tokens past those it was made for are attended one by
+ * one, or come out as zeros where they fall into a group that shares a prefix;
+ * a buffer of that size that holds no plan is not used.  No counterpart in the
+ * reference: flashinfer plans its own decode batches
+ * (python/flashrec/attention/flashinfer.py:262-349). */
 int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t Hk);
 int fr_paged_attention_plan(const int32_t* kv_indices, const int32_t* kv_start, const int32_t* kv_len,
                             int64_t T, int64_t Hq, int64_t Hk, int32_t* group_prefix, void* stream);
