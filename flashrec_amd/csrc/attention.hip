@@ -21,8 +21,8 @@
 // over NW waves of a workgroup when the items alone do not fill the chip.
 // Arithmetic in fp32 (e4m3 and bf16 convert exactly); the probabilities of
 // whole groups are rounded to bf16 (as the reference's bf16 SDPA does), those
-// of groups in several segments are carried as two bf16 terms (16 significant
-// bits).  Output bf16.
+// of groups in several segments keep their fp32 value, as three bf16 terms.
+// Output bf16.
 #include <type_traits>
 
 #include "attn_plan.h"
@@ -195,7 +195,7 @@ struct Softmax {
 
 // Block range [part * blocks / parts, (part + 1) * blocks / parts) of a
 // segment, for the queries of its tokens (the other columns' results mean
-// nothing).  FINE: probabilities as two bf16 terms, and `nan` reports a NaN
+// nothing).  FINE: probabilities as three bf16 terms, and `nan` reports a NaN
 // code in a V row that some of the segment's queries must not see (its product
 // with their zero probability would still be NaN).  `stage`: kStage bytes of
 // this wave's LDS.
@@ -341,20 +341,25 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, uint8_t* stage
       pr[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[v], a.qscale, -mref));  // x = -inf gives 0
       X.l += pr[v];
     }
-    bf16x8_t pb[2], pl[2];
+    // FINE: three terms of 8 significant bits hold all 24 of the fp32
+    // probability (each difference is exact)
+    constexpr int TERMS = FINE ? 3 : 1;
+    bf16x8_t pb[2][TERMS];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      u32x4 w, lo;
+    for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        w[t] = pack_bf16x2(pr[8 * c + 2 * t], pr[8 * c + 2 * t + 1]);
-        if constexpr (FINE)
-          lo[t] = pack_bf16x2(pr[8 * c + 2 * t] - __uint_as_float(w[t] << 16),
-                              pr[8 * c + 2 * t + 1] - __uint_as_float(w[t] & 0xFFFF0000u));
+      for (int k = 0; k < TERMS; ++k) {
+        u32x4 w;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          float& p0 = pr[8 * c + 2 * t];
+          float& p1 = pr[8 * c + 2 * t + 1];
+          w[t] = pack_bf16x2(p0, p1);
+          p0 -= __uint_as_float(w[t] << 16);
+          p1 -= __uint_as_float(w[t] & 0xFFFF0000u);
+        }
+        pb[c][k] = __builtin_bit_cast(bf16x8_t, w);
       }
-      pb[c] = __builtin_bit_cast(bf16x8_t, w);
-      if constexpr (FINE) pl[c] = __builtin_bit_cast(bf16x8_t, lo);
-    }
     // O^T += V^T . P^T; A[dim][k] through the transposing LDS read
     const int g = lane >> 4, i16 = lane & 15;
 #pragma unroll
@@ -368,15 +373,16 @@ __device__ __forceinline__ void attend_segment(const AttnArgs& a, uint8_t* stage
             __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(vs + (r0 + 8) * kVRow + 2 * col));
         const bf16x8_t av = __builtin_bit_cast(
             bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        X.O[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pb[c], X.O[mt], 0, 0, 0);
-        if constexpr (FINE) X.O[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pl[c], X.O[mt], 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < TERMS; ++k)
+          X.O[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, pb[c][k], X.O[mt], 0, 0, 0);
       }
     }
   };
 
   if (b0 >= b1) return;
   // the next block's gathers are in flight while a block is multiplied; the
-  // two-term form has no registers to spare for them
+  // three-term form has no registers to spare for them
   constexpr bool AHEAD = !FINE;
   int32_t slot = slot_of(b0);
   if (AHEAD) {

@@ -115,3 +115,31 @@ def test_wave_rule():
     w = load().fr_paged_attention_waves
     assert w(4096, 16, 8, 4096 * 131) == 1 and w(0, 16, 8, 0) == 1 and w(10, 15, 4, 10) == 1
     assert w(50, 16, 8, 50 * 202) > 1 and w(1999, 16, 8, 1999) > 1
+
+
+@pytest.mark.parametrize("waves", [1, 4])
+@pytest.mark.parametrize("hq,hk", [(16, 8), (8, 8), (16, 4), (16, 2)])
+def test_probabilities_keep_32_bits(dev, hq, hk, waves):
+    """Tokens with lists of their own: the difference of two nearly equal
+    probabilities, times 448.  It is 2^-11 of them and more, so an error of
+    2^-17 in each, which 16 bits leave, is up to 2^-5 of the result, where
+    32-bit scores, powers and sums leave about 2^-10; the output rounds by 2^-8."""
+    print(f"probabilities {hq}/{hk}, {waves} waves", flush=True)
+    t = 70
+    g = torch.Generator().manual_seed(11)
+    k = torch.zeros(4, hk, 128)
+    k[1:3, :, 0] = torch.tensor([1.0, 1.125])[:, None]
+    k[3, :, 1] = 1.0
+    v = torch.tensor([0.0, 448.0, -448.0, 0.0])[:, None, None].expand(4, hk, 128).contiguous()
+    q = torch.zeros(t, hq, 128)
+    q[:, :, 0] = 0.05 + 0.15 * torch.rand(t, hq, generator=g)
+    q[:, :, 1] = 8 * torch.randn(t, hq, generator=g)
+    q = q.to(torch.bfloat16)
+    idx = torch.tensor([1, 2, 3], dtype=torch.int32).repeat(t)
+    start, lens = torch.arange(t, dtype=torch.int32) * 3, torch.full((t,), 3, dtype=torch.int32)
+    got = _run(dev, q, k.to(E4M3), v.to(E4M3), idx, start, lens, waves, True).double()
+    a, c = q[..., 0].double(), q[..., 1].double()
+    p = torch.softmax(torch.stack([a, 1.125 * a, c], -1) * SCALE, -1)
+    want = ((p[..., 0] - p[..., 1]) * 448)[..., None]
+    err = ((got - want) / want).abs().max().item()
+    assert err < 2.0 ** -8 + 2.0 ** -9, err
