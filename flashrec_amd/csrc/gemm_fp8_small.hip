@@ -193,8 +193,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_fp8_small(GemmArgs g, int out_dt
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  // one slot's loads, then the next one's: the counted waits name them by
+  // their place in issue order
 #pragma unroll
-  for (int q = 0; q < NS; ++q) issue(q, s0 + q);
+  for (int q = 0; q < NS; ++q) {
+    issue(q, s0 + q);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   fetch_scales();
   for (int s = s0; s < s1; s += NS) {
     slot(std::integral_constant<int, 0>{});
