@@ -432,14 +432,18 @@ __global__ __launch_bounds__(256) void row_kernel_split(RowArgs a) {
   }
 }
 
-// fp16 and fp32 rows: one 256-thread workgroup per row, each lane with NC
-// chunks of 8 elements held in registers (chunk c at column (256 c + tid) *
-// 8), so the row is read once with 16-byte loads.  The generic kernel's one
-// wave re-reads it per pass, two or four bytes a lane, and its latency is the
-// launch's: fp16 SiLU + quant of 13 rows x 12288 69.1 -> 6.4 us, of 1001 rows
-// 89.5 -> 16.3; add + RMSNorm of 13 rows x 2048 29.4 -> 4.3, of 1001 29.2 ->
-// 6.7.  The generic kernel's arithmetic (torch's formulas, IEEE division) but
-// for the order of the sum of squares.
+// fp16 and fp32 rows: WPR waves per row (4: a 256-thread workgroup, 1: four
+// rows a workgroup), each lane with NC chunks of 8 elements held in registers
+// (chunk c at column (64 WPR c + lane of the row) * 8), so the row is read once
+// with 16-byte loads.  The generic kernel's one wave re-reads it per pass, two
+// or four bytes a lane, and its latency is the launch's: fp16 SiLU + quant of 13
+// rows x 12288 69.1 -> 6.4 us, of 1001 rows 89.5 -> 16.3; add + RMSNorm of 13
+// rows x 2048 29.4 -> 4.3, of 1001 29.2 -> 6.7.  The generic kernel's arithmetic
+// (torch's formulas, IEEE division) but for the order of the sum of squares.
+// Rows up to 1024 wide take one wave: they leave half and more of a workgroup's
+// lanes without a chunk, which cost as much as the others (fp16 SiLU + quant of
+// 16384 x 512: generic 25.6, a workgroup a row 36.2, a wave a row 15.7; RMSNorm +
+// quant of 65536 x 256: 42.1, 75.0, 32.5).
 template <int DT>
 __device__ __forceinline__ void load8(const typename Elem<DT>::T* p, float* f) {
   if constexpr (DT == FR_DTYPE_FP32) {
@@ -471,17 +475,19 @@ __device__ __forceinline__ void store8(typename Elem<DT>::T* p, const float* f) 
   }
 }
 
-template <int MODE, int DT, int NC, bool QOUT>
+template <int MODE, int DT, int NC, bool QOUT, int WPR>
 __global__ __launch_bounds__(256) void row_kernel_fine(RowArgs a) {
   using E = Elem<DT>;
   using T = typename E::T;
   constexpr bool kNorm = MODE == kRms || MODE == kAddRms;
+  static_assert(WPR == 1 || WPR == 4, "a wave or a workgroup per row");
   __shared__ float red[2][4];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int64_t row = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t row = WPR == 1 ? static_cast<int64_t>(blockIdx.x) * 4 + wave : blockIdx.x;
+  if (WPR == 1 && row >= a.M) return;  // (no barrier below for one wave per row)
+  const int tid = WPR == 1 ? lane : threadIdx.x;  // of the row's threads
   const int64_t K = a.K;
-  auto col = [&](int c) __attribute__((always_inline)) { return (static_cast<int64_t>(c) * 256 + tid) * 8; };
+  auto col = [&](int c) __attribute__((always_inline)) { return (static_cast<int64_t>(c) * (64 * WPR) + tid) * 8; };
   const T* const xr = reinterpret_cast<const T*>(a.x) + row * a.ldx;
   float v[NC][8], o[NC][8];  // o: the residual, the norm weight or the up half
 #pragma unroll
@@ -503,9 +509,11 @@ __global__ __launch_bounds__(256) void row_kernel_fine(RowArgs a) {
   }
   if (MODE == kSilu) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+    for (int c = 0; c < NC; ++c) {
+      if (col(c) >= K) continue;
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[c][i] = E::round(E::round(silu_any<DT>(v[c][i])) * o[c][i]);
+    }
   }
   if (kNorm) {
 #pragma unroll
@@ -517,9 +525,11 @@ __global__ __launch_bounds__(256) void row_kernel_fine(RowArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) ss += v[c][i] * v[c][i];
     ss = wave_sum(ss);
-    if (lane == 0) red[0][wave] = ss;
-    __syncthreads();
-    ss = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    if constexpr (WPR > 1) {
+      if (lane == 0) red[0][wave] = ss;
+      __syncthreads();
+      ss = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    }
     const float rstd = 1.0f / __builtin_sqrtf(ss / static_cast<float>(K) + a.eps);
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -541,9 +551,12 @@ __global__ __launch_bounds__(256) void row_kernel_fine(RowArgs a) {
       for (int i = 0; i < 8; ++i) amax = maxnan(amax, __builtin_fabsf(v[c][i]));
     }
   amax = wave_maxnan(amax);
-  if (lane == 0) red[1][wave] = amax;
-  __syncthreads();
-  amax = maxnan(maxnan(maxnan(red[1][0], red[1][1]), maxnan(red[1][2], red[1][3])), kAmaxFloor);
+  if constexpr (WPR > 1) {
+    if (lane == 0) red[1][wave] = amax;
+    __syncthreads();
+    amax = maxnan(maxnan(red[1][0], red[1][1]), maxnan(red[1][2], red[1][3]));
+  }
+  amax = maxnan(amax, kAmaxFloor);
   const float scale = amax / kFp8Max;
   if (tid == 0) a.s[row] = scale;
   uint8_t* const qrow = a.q + row * a.ldq;
@@ -561,11 +574,12 @@ __global__ __launch_bounds__(256) void row_kernel_fine(RowArgs a) {
 
 template <int MODE, int DT, bool QOUT>
 static hipError_t launch_fine(const RowArgs& a, hipStream_t st) {
-  const int64_t nc = (a.K + 2047) / 2048;
-  const dim3 grid(static_cast<unsigned>(a.M));
-  if (nc <= 1) hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 1, QOUT>), grid, dim3(256), 0, st, a);
-  else if (nc <= 2) hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 2, QOUT>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 4, QOUT>), grid, dim3(256), 0, st, a);
+  const dim3 one(static_cast<unsigned>(a.M)), four(static_cast<unsigned>((a.M + 3) / 4));
+  if (a.K <= 512) hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 1, QOUT, 1>), four, dim3(256), 0, st, a);
+  else if (a.K <= 1024) hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 2, QOUT, 1>), four, dim3(256), 0, st, a);
+  else if (a.K <= 2048) hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 1, QOUT, 4>), one, dim3(256), 0, st, a);
+  else if (a.K <= 4096) hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 2, QOUT, 4>), one, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((row_kernel_fine<MODE, DT, 4, QOUT, 4>), one, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
@@ -624,14 +638,22 @@ static int launch_rows(RowArgs a, int dtype, hipStream_t st) {
   if (MODE == kRms || MODE == kAddRms) vec = vec && al16(a.w);
   if (QOUT) vec = vec && a.ldq % 8 == 0 && (reinterpret_cast<uintptr_t>(a.q) & 7u) == 0;
   else vec = vec && a.ldq % 8 == 0 && al16(a.q);
-  // fp16 / fp32 rows of whole aligned 8-element chunks
+  // fp16 / fp32 rows of whole aligned 8-element chunks; a launch holds less than
+  // 2^32 threads, so more rows than a workgroup each allows go by waves
   const int64_t esz = dtype == FR_DTYPE_FP32 ? 4 : 2;
-  bool fine = (dtype == FR_DTYPE_FP16 || dtype == FR_DTYPE_FP32) && K % 8 == 0 && K <= 8192 && a.M <= 0x7FFFFFFF &&
-              (a.ldx * esz) % 16 == 0 && al16(a.x);
+  bool fine = (dtype == FR_DTYPE_FP16 || dtype == FR_DTYPE_FP32) && K % 8 == 0 && K <= 8192 &&
+              (K <= 1024 || a.M < (int64_t(1) << 24)) && (a.ldx * esz) % 16 == 0 && al16(a.x);
   if (MODE == kAddRms) fine = fine && (a.ldr * esz) % 16 == 0 && al16(a.res);
   if (MODE == kRms || MODE == kAddRms) fine = fine && al16(a.w);
   if (QOUT) fine = fine && a.ldq % 8 == 0 && (reinterpret_cast<uintptr_t>(a.q) & 7u) == 0;
   else fine = fine && (a.ldq * esz) % 16 == 0 && al16(a.q);
+  // Narrow rows leave lanes of row_kernel_fine without a chunk, where the generic
+  // kernel's lanes take two or four bytes each of any width.  us, generic / fine:
+  // fp16 quant 32768 x 128 10.0 / 12.0, 8192 x 256 5.7 / 5.1; SiLU + quant 32768 x
+  // 128 15.4 / 25.2, x 256 26.4 / 26.1.  SiLU alone is bound by its divisions, so
+  // lanes without a second chunk cost it most: 32768 x 256 13.7 / 19.7, x 640
+  // 27.2 / 35.4, x 512 22.5 / 20.9, 2048 x 640 5.1 / 4.9.
+  fine = fine && K >= 256 && !(MODE == kSilu && !QOUT && K < 1024 && K != 512 && a.M > 2048);
   hipError_t err;
   if (fine) {
     err = dtype == FR_DTYPE_FP16 ? launch_fine<MODE, FR_DTYPE_FP16, QOUT>(a, st)

@@ -74,3 +74,27 @@ def test_aligned_rows_match_unaligned(dev, k, dtype):
             else:  # scales, as bits; NaN payloads are not pinned
                 fa, fb = a.view(torch.float32), b.view(torch.float32)
                 assert bool(((a == b) | (fa.isnan() & fb.isnan())).all()), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("k", [64, 504, 512, 520, 1016, 1024, 1032])
+def test_narrow_rows_match_unaligned(dev, k, dtype):
+    """The same at the edges of the widths that take a wave per row (9 rows: two
+    workgroups of four and one of one)."""
+    test_aligned_rows_match_unaligned(dev, k, dtype)
+
+
+def test_more_rows_than_workgroups(dev):
+    """Past 2^24 rows: a workgroup of 256 threads for each would be more than a
+    launch holds."""
+    from flashrec_amd.kernel.sglops import per_token_quant_fp8
+
+    m = (1 << 24) + 5
+    x = torch.zeros(m, 8, dtype=torch.float16, device=dev)
+    x[-3:] = torch.arange(8, device=dev)
+    q, s = per_token_quant_fp8(x)
+    want = torch.full((m,), 1e-12, device=dev)
+    want[-3:] = 7.0
+    assert torch.equal(s.view(-1), want / 448)
+    assert bool((q[:-3].view(torch.uint8) == 0).all()) and torch.equal(
+        q[-1].float(), (torch.arange(8, device=dev) / s[-1]).to(torch.float8_e4m3fn).float())
