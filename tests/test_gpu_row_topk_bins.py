@@ -46,3 +46,10 @@ def test_row_topk_bins(dev, v, c, kind):
     check(row_topk(x.to(dev), c), x)
     if kind != "masked":  # (a row's log-probabilities as the log-softmax kernel writes them)
         check(row_topk(x.to(dev), c, log_softmax=True), log_softmax_f32(x.to(dev)).cpu())
+
+
+@pytest.mark.parametrize("kind", ["both", "one", "outlier", "masked", "zeros"])
+@pytest.mark.parametrize("v,c", [(16384, 1024), (16384, 40), (2048, 700)])
+def test_row_topk_bins_widest(dev, v, c, kind):
+    """64 keys a thread (two words of boundary-bin bits) and 8."""
+    test_row_topk_bins(dev, v, c, kind)
