@@ -37,6 +37,7 @@
 // 18.2 + 18.3 so; 1 x 512 33.6 + 33.7 -> 15.4 + 17.8; 8 x 35 21.4 + 10.6 -> 10.1
 // + 8.4.  What is left is latency: kernel 2 is one CU per request.
 #include <mutex>
+#include <type_traits>
 
 #include "fr_common.h"
 
@@ -210,12 +211,10 @@ struct ListAt {
 __device__ __forceinline__ void sort_desc(uint64_t* keys, int n, uint64_t* buf, SelectLds& L) {
   const int t = threadIdx.x;
   const uint64_t key[1] = {t < n ? keys[t] : 0};
-  if (n <= 64) {  // one wave, in registers
+  if (n <= 64) {  // one wave, in registers; a network as wide as the keys
     if (t < 64) {
       uint64_t v = key[0];
-#pragma unroll
-      for (int k = 2; k <= 64; k <<= 1)
-#pragma unroll
+      for (int k = 2; k < 2 * n; k <<= 1)
         for (int j = k >> 1; j > 0; j >>= 1) {
           const uint64_t o = shfl_xor_u64(v, j);
           const bool want_max = ((t & j) == 0) == ((t & k) == 0);
@@ -301,8 +300,10 @@ __global__ __launch_bounds__(64 * kSliceWaves) void genrec_slice_topk(GenrecArgs
   // lookups are issued, then the chunks are compacted in order (ballot prefix
   // sums, stopping at K): two memory round trips per group.  Loads are
   // unconditional on clamped indices: under a lane's condition each would
-  // wait for the one before it.
-  constexpr int kPre = 16;
+  // wait for the one before it.  Narrow beams take groups of one or four chunks:
+  // the instructions of sixteen, and of sixteen keys a thread in kernel 2, were
+  // most of a small step (both kernels: 1 beam of 16 candidates 13.8 -> 8.1 us, 20
+  // beams of 40 21.6 -> 15.3).
   if (wave < nb) {
     const int b = b0 + wave;
     const float cb = a.cum[static_cast<int64_t>(n) * a.BW + b];
@@ -319,7 +320,8 @@ __global__ __launch_bounds__(64 * kSliceWaves) void genrec_slice_topk(GenrecArgs
     if (staged && 16 * lane < a.vsz)
       *reinterpret_cast<u32x4*>(rows[wave] + 16 * lane) = *reinterpret_cast<const u32x4*>(allow + 16 * lane);
     int count = 0;
-    for (int g0 = 0; g0 < a.C && count < a.K; g0 += 64 * kPre) {
+    auto group = [&](int g0, auto pre_c) __attribute__((always_inline)) {
+      constexpr int kPre = decltype(pre_c)::value;
       float v[kPre];
       int64_t rel[kPre];
 #pragma unroll
@@ -349,7 +351,11 @@ __global__ __launch_bounds__(64 * kSliceWaves) void genrec_slice_topk(GenrecArgs
         if (ok && pos < a.K) buf[wave * a.K + pos] = make_key(v[u], static_cast<uint32_t>(b * a.C + c));
         count += __builtin_popcountll(bal);
       }
-    }
+    };
+    if (a.C <= 64) group(0, std::integral_constant<int, 1>{});
+    else if (a.C <= 256) group(0, std::integral_constant<int, 4>{});
+    else
+      for (int g0 = 0; g0 < a.C && count < a.K; g0 += 1024) group(g0, std::integral_constant<int, 16>{});
     if (lane == 0) len[wave] = count < a.K ? count : a.K;
   } else if (lane == 0) {
     len[wave] = 0;
@@ -389,45 +395,50 @@ __global__ __launch_bounds__(1024) void genrec_request_topk_expand(GenrecArgs a)
   const int n = blockIdx.x;
   const int K = a.K;
   const uint64_t* lists = a.scratch + static_cast<int64_t>(n) * a.S * (1 + K);
-  // The slices' lists go in groups of G that fill the threads' registers; the
-  // keys kept from the groups before ride along.
-  constexpr int kPer = 16;
-  const int G = kPer * 1024 / K < 64 ? kPer * 1024 / K : 64;  // (len[] holds 64)
+  // The slices' lists go in groups of G that fill the threads' registers (one
+  // key a thread where that holds all of them); the keys kept from the groups
+  // before ride along.
   // keys kept: up to twice K's power of two, so that one histogram pass mostly
   // does and the sort below stays short
   int cap = 2;
   while (cap < K) cap <<= 1;
   cap = cap < 512 ? 2 * cap : 1024;
   int held = 0;
-  for (int g0 = 0; g0 < a.S; g0 += G) {
-    const int gs = a.S - g0 < G ? a.S - g0 : G;
-    const uint64_t* gl = lists + static_cast<int64_t>(g0) * (1 + K);
-    if (threadIdx.x == 0) cursor = 0;
-    uint64_t key[kPer + 1];
-    ListAt at(K);
+  auto select = [&](auto per_c) __attribute__((always_inline)) {
+    constexpr int kPer = decltype(per_c)::value;
+    const int G = kPer * 1024 / K < 64 ? kPer * 1024 / K : 64;  // (len[] holds 64)
+    for (int g0 = 0; g0 < a.S; g0 += G) {
+      const int gs = a.S - g0 < G ? a.S - g0 : G;
+      const uint64_t* gl = lists + static_cast<int64_t>(g0) * (1 + K);
+      if (threadIdx.x == 0) cursor = 0;
+      uint64_t key[kPer + 1];
+      ListAt at(K);
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const uint64_t x = gl[at.l < gs ? static_cast<uint32_t>(at.l * (1 + K) + 1 + at.i) : 0u];
-      key[r] = at.l < gs ? x : 0;
-      at.next(K);
+      for (int r = 0; r < kPer; ++r) {
+        const uint64_t x = gl[at.l < gs ? static_cast<uint32_t>(at.l * (1 + K) + 1 + at.i) : 0u];
+        key[r] = at.l < gs ? x : 0;
+        at.next(K);
+      }
+      if (threadIdx.x < 64)
+        len[threadIdx.x] = static_cast<int>(threadIdx.x) < gs ? static_cast<int>(gl[threadIdx.x * (1 + K)]) : 0;
+      __syncthreads();
+      key[kPer] = static_cast<int>(threadIdx.x) < held ? acc[threadIdx.x] : 0;
+      int total = len[threadIdx.x & 63];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+      total += held;
+      __syncthreads();  // acc, len and the cursor are read
+      const uint64_t least = select_top<kPer + 1>(key, total, K, cap, sel);
+#pragma unroll
+      for (int r = 0; r <= kPer; ++r)
+        if (key[r] != 0 && key[r] >= least) acc[atomicAdd(&cursor, 1u)] = key[r];
+      __syncthreads();
+      held = static_cast<int>(cursor);
+      __syncthreads();
     }
-    if (threadIdx.x < 64)
-      len[threadIdx.x] = static_cast<int>(threadIdx.x) < gs ? static_cast<int>(gl[threadIdx.x * (1 + K)]) : 0;
-    __syncthreads();
-    key[kPer] = static_cast<int>(threadIdx.x) < held ? acc[threadIdx.x] : 0;
-    int total = len[threadIdx.x & 63];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
-    total += held;
-    __syncthreads();  // acc, len and the cursor are read
-    const uint64_t least = select_top<kPer + 1>(key, total, K, cap, sel);
-#pragma unroll
-    for (int r = 0; r <= kPer; ++r)
-      if (key[r] != 0 && key[r] >= least) acc[atomicAdd(&cursor, 1u)] = key[r];
-    __syncthreads();
-    held = static_cast<int>(cursor);
-    __syncthreads();
-  }
+  };
+  if (a.S * K <= 1024) select(std::integral_constant<int, 1>{});
+  else select(std::integral_constant<int, 16>{});
   sort_desc(acc, held, reinterpret_cast<uint64_t*>(sel_parent), sel);
   const uint64_t* res = acc;
   const int got = held < K ? held : K;

@@ -40,3 +40,12 @@ def test_infinite_scores_unmasked(dev):
     args[1] = torch.sort(lp, dim=-1, descending=True).values
     _compare(dev, tuple(args), 48, apply_mask=False)
     _compare(dev, tuple(args), 48)
+
+
+@pytest.mark.parametrize("n,bw,c,k", [(2, 3, 64, 2), (1, 17, 65, 32), (1, 20, 256, 33), (2, 20, 257, 63), (1, 16, 1024, 1024),
+                                      (1, 17, 64, 512), (1, 32, 40, 513), (1, 1030, 1, 1), (3, 1100, 2, 17)])
+def test_narrow_beams_and_few_lists(dev, n, bw, c, k):
+    """Candidates a beam around one and four chunks of 64, slices' lists around
+    1024 keys in all (17 and 32 beams are two slices), more lists than a group."""
+    print(f"narrow {n}x{bw}x{c} top {k}", flush=True)
+    _compare(dev, _case(n, bw, c, 768, 20, 0.8, 13 * bw + c), k)
