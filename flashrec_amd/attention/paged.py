@@ -120,6 +120,10 @@ class AttentionBackend:
             nidx = int(kv.numel())
             if nidx > 0 and kv.data_ptr() != bufs["indices"].data_ptr():
                 bufs["indices"][:nidx].copy_(kv, non_blocking=True)
+            # (no "entries": a captured launch serves every length its buffers
+            # hold, so its split is chosen for their capacity.  us, 16/8 heads:
+            # 2048 x 130 in rows of 4096 slots 21.5 for 19.6 unsplit, where 1248 x
+            # 1133 unsplit would take 180 for 73)
             return {"indices": bufs["indices"], "start": bufs["indptr"][:n], "len": bufs["kv_len"][:n]}
         indptr = batch.kv_indptr
         if indptr is None:
@@ -144,8 +148,13 @@ class AttentionBackend:
                 length.append(int(prefix[i]) + j + 1)
             off += seq[i]
         kv = batch.kv_indices.view(-1).to(device=self.device, dtype=torch.int32).contiguous()
+        # for the split of the keys over waves: tokens that share their prompt's
+        # list count one slot each (so that a long cached prefix is not taken for
+        # lists of their own), else each reads its own
+        shared = len(start) >= 8 * n
         return {
             "indices": kv,
+            "entries": len(start) if shared else sum(length),
             "start": torch.tensor(start, dtype=torch.int32).to(self.device),
             "len": torch.tensor(length, dtype=torch.int32).to(self.device),
         }
@@ -162,7 +171,8 @@ class AttentionBackend:
             raise RuntimeError("AttentionBackend.forward before prepare() (kv_indices required)")
         return paged_attention(q, self.kv_pool.k_cache(layer_id), self.kv_pool.v_cache(layer_id),
                                self._plan["indices"], self._plan["start"], self._plan["len"],
-                               self.scale, group_prefix=self._plan.get("group_prefix"))
+                               self.scale, group_prefix=self._plan.get("group_prefix"),
+                               entries=self._plan.get("entries"))
 
 
     @torch.compiler.disable
@@ -174,7 +184,8 @@ class AttentionBackend:
             raise RuntimeError("AttentionBackend.forward_quant_fp8 before prepare() (kv_indices required)")
         return paged_attention_quant_fp8(q, self.kv_pool.k_cache(layer_id), self.kv_pool.v_cache(layer_id),
                                          self._plan["indices"], self._plan["start"], self._plan["len"],
-                                         self.scale, group_prefix=self._plan.get("group_prefix"))
+                                         self.scale, group_prefix=self._plan.get("group_prefix"),
+                                         entries=self._plan.get("entries"))
 
 
 def plan_size(T: int, hq: int, hk: int) -> int:
@@ -262,6 +273,10 @@ def _check_plan(group_prefix: Optional[torch.Tensor], T: int, hq: int, hk: int) 
     return group_prefix.data_ptr() if records else 0
 
 
+def _waves(T: int, hq: int, hk: int, kv_indices: torch.Tensor, entries: Optional[int]) -> int:
+    return int(load().fr_paged_attention_waves(T, hq, hk, kv_indices.numel() if entries is None else int(entries)))
+
+
 def _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len):
     require_device(q, k_cache, v_cache, kv_indices, kv_start, kv_len)
     if q.dtype != torch.bfloat16:
@@ -285,8 +300,8 @@ def _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len):
 def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                               kv_indices: torch.Tensor, kv_start: torch.Tensor, kv_len: torch.Tensor,
                               scale: float, group_prefix: Optional[torch.Tensor] = None,
-                              out: Optional[torch.Tensor] = None, out_scale: Optional[torch.Tensor] = None
-                              ) -> Tuple[torch.Tensor, torch.Tensor]:
+                              out: Optional[torch.Tensor] = None, out_scale: Optional[torch.Tensor] = None,
+                              entries: Optional[int] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """``per_token_quant_fp8(paged_attention(...).reshape(T, -1))`` in one
     kernel: the o projection's e4m3 input ``[T, Hq * D]`` and its scales
     ``[T, 1]`` (qwen3.py:131-134 -> linear.py:118-151), bit-for-bit the two
@@ -307,7 +322,7 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     # where paged_attention splits its items' keys over waves, the quant runs
     # on its rows (one more launch of 3 us; 512 rows over 1503 keys take 89 us
     # fused and unsplit, 25 us so)
-    if int(load().fr_paged_attention_waves(T, Hq, Hk, kv_indices.numel())) == 1:
+    if _waves(T, Hq, Hk, kv_indices, entries) == 1:
         try:
             call("fr_paged_attention_quant_fp8",
                  q.data_ptr(), q.stride(0), q.stride(1),
@@ -319,7 +334,8 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
             return out, out_scale
         except Unsupported:
             pass
-    o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, group_prefix=group_prefix)
+    o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, group_prefix=group_prefix,
+                        entries=entries)
     codes = out if out.is_contiguous() else torch.empty((T, Hq * D), dtype=out.dtype, device=out.device)
     call("fr_per_token_quant_fp8", o.data_ptr(), DTYPE_CODE[o.dtype], T, Hq * D, Hq * D, codes.data_ptr(),
          out_scale.data_ptr(), stream_of(q))
@@ -331,13 +347,17 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                     kv_indices: torch.Tensor, kv_start: torch.Tensor, kv_len: torch.Tensor,
                     scale: float, out: Optional[torch.Tensor] = None,
-                    group_prefix: Optional[torch.Tensor] = None) -> torch.Tensor:
+                    group_prefix: Optional[torch.Tensor] = None, entries: Optional[int] = None) -> torch.Tensor:
     """softmax(q k^T * scale) v over each query token's slot list.
 
     q: [T, Hq, 128] bf16 (unit inner stride); k_cache / v_cache: [slots, Hk,
     128] float8_e4m3fn; kv_indices / kv_start / kv_len: int32 on the device.
     group_prefix: the plan of ``attention_plan`` for the same slot lists, or
-    None (each call then finds the shared prefixes itself).
+    None (each call then finds the shared prefixes itself).  entries: the slots
+    that the tokens' lists hold together, which decides over how many waves the
+    keys of a query group are split (and so the order of its sums); without it
+    the length of kv_indices is taken, and with a buffer longer than its lists
+    the capacity counts.
     """
     T, Hq, D, slots, Hk = _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len)
     if out is None:
@@ -349,5 +369,5 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
          slots, kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
          out.data_ptr(), out.stride(0), out.stride(1),
          T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk),
-         int(load().fr_paged_attention_waves(T, Hq, Hk, kv_indices.numel())), stream_of(q))
+         _waves(T, Hq, Hk, kv_indices, entries), stream_of(q))
     return out

@@ -55,3 +55,26 @@ def test_what_a_plan_may_be():
                 torch.zeros(8, dtype=torch.int32)[::2]):
         with pytest.raises(ValueError, match="plan"):
             paged._check_plan_buffer(bad, 4, paged._plan_records(bad, 4, stride))
+
+
+def test_split_of_prompts_over_cached_prefixes():
+    """A prompt that continues a long cached prefix is split like one without;
+    prompts of a token each are split as decode rows are."""
+    from types import SimpleNamespace
+
+    from flashrec_amd._lib import load
+    from flashrec_amd.attention.paged import AttentionBackend
+
+    be = AttentionBackend(SimpleNamespace(device=torch.device("cpu")), 16, 8, 128)
+
+    def waves(prompts):  # (cached, new) of each
+        seq = torch.tensor([c + e for c, e in prompts], dtype=torch.int32)
+        plan = be._plan_prefill(SimpleNamespace(
+            n_rows=len(prompts), seq_lens_cpu=seq, extend_seq_lens=[e for _, e in prompts],
+            extend_prefix_lens=[c for c, _ in prompts], kv_indices=torch.zeros(int(seq.sum()), dtype=torch.int32)))
+        return load().fr_paged_attention_waves(int(plan["start"].numel()), 16, 8, plan["entries"])
+
+    assert waves([(0, 100)]) == waves([(1500, 100)])
+    assert waves([(0, 1100)]) == waves([(9000, 1100)]) > 1
+    assert waves([(0, 300)] * 4) == waves([(3000, 300)] * 4) > 1
+    assert waves([(129, 1)] * 2048) == load().fr_paged_attention_waves(2048, 16, 8, 2048 * 130)
