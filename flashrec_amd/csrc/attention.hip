@@ -533,6 +533,10 @@ struct Segments {
       if (whole == 0) linked = linked_tokens<TOK>(a, t0, ntok, lane);
     }
   }
+  // Segments of the group (as far as the record knows its tokens).
+  __device__ __forceinline__ int number(int lane) const {
+    return planned ? __builtin_popcountll(__ballot(lane < ntok && cnt > 0)) : ntok - __builtin_popcount(linked);
+  }
   __device__ __forceinline__ Segment at(const AttnArgs& a, int first, const Query& Q, bool single, int lane) const {
     if (single) return Segment{first, 1, 0, true};
     const int tok = (lane & 31) / NREP;
@@ -688,7 +692,39 @@ __global__ __launch_bounds__(64 * NW, 2) void paged_attn_split_d128(AttnArgs a) 
     merge(Segment{0, 32 / NREP, 0, false}, X);  // tokens that the plan did not know: zeros
     return;
   }
+  // Several segments.  As many as waves and more go to the waves in turn, each
+  // on one wave and without a merge: rows with lists of their own else pay three
+  // barriers and a merge for a block or two of each wave.  16/8 heads, us, split
+  // / dealt: 64 rows x 40 keys 79.2 / 26.4 (66.7 token by token on the VALU),
+  // 64 x 200 114 / 59.2, 64 x 1500 291 / 219.
   int single_until = 0;
+  if (segs.number(lane) >= NW) {
+    const int tok = n / NREP;
+    int dealt = 0;
+    bool mine = false;
+    for (int at = 0; at < segs.ntok;) {
+      const bool single = at < single_until;
+      const Segment s = segs.at(a, at, Q, single, lane);
+      if (!single) mine = dealt++ % NW == wave;  // (a segment taken again stays with its wave)
+      if (mine) {
+        nan = false;
+        attend_segment<NREP, true>(a, stage, kh, lane, Q, s, 0, 1, X, nan);
+        if (nan && s.count > 1) {
+          single_until = at + s.count;
+          continue;
+        }
+        const float lt = X.l + __shfl_xor(X.l, 32, 64);
+        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+        if (tok >= at && tok < at + s.count) {
+          uint16_t* const op = a.out + (t0 + tok) * a.sot + (kh * NREP + n % NREP) * a.soh;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) *reinterpret_cast<u32x2*>(op + 8 * i + 4 * h) = out4(X, inv, i >> 2, i & 3);
+        }
+      }
+      at += s.count;
+    }
+    return;
+  }
   for (int at = 0; at < segs.ntok;) {
     if (threadIdx.x == 0) saw_nan = 0;
     __syncthreads();  // the last merge has been read, the flag is clear
@@ -791,13 +827,16 @@ __global__ __launch_bounds__(512, 1) void paged_attn_grouped_quant_d128(AttnArgs
 //   4096 x 130 (2048)       21.9 /    - / 46.4 / 74.3    4096 x 1002  72.7 / 85.3 / 91.1 / 127
 //   prefill 1999 (1000)     76.9 / 47.9 / 44.5 / 60.3    4 x 500 (1000)  33.1 / 30.3 / 30.4 / 41.5
 //   prefill 4000 (2000)      159 /  122 /  125 /  159
-static int attn_waves(int64_t T, int64_t items, int64_t entries) {
+// A kv head per query head makes groups of 32 tokens, whose segments gain most
+// from being dealt to waves (attention alone): 1024 rows x 200, a list each, 32/32
+// heads 542 / 398 / 393 / 415; 8 requests x 512 beams x 132, 8/8 heads 18.5 / 18.7.
+static int attn_waves(int64_t T, int64_t items, int64_t entries, int64_t nrep) {
   const int64_t simds = 4 * num_cus();
   const bool prompt = entries < 8 * T;
   const int64_t keys = entries / T;
   if (4 * items <= simds) return prompt || keys > 600 ? 8 : 4;
   if (2 * items <= simds) return 4;
-  if (items <= simds) return prompt ? 4 : (keys < 300 ? 1 : (4 * items <= 3 * simds ? 4 : 2));
+  if (items <= simds) return prompt ? 4 : (keys < 300 ? (nrep == 1 ? 2 : 1) : (4 * items <= 3 * simds ? 4 : 2));
   return prompt && items <= 2 * simds ? 2 : 1;
 }
 
@@ -947,7 +986,7 @@ extern "C" int64_t fr_paged_attention_plan_size(int64_t T, int64_t Hq, int64_t H
 
 extern "C" int fr_paged_attention_waves(int64_t T, int64_t Hq, int64_t Hk, int64_t entries) {
   const int64_t groups = attn_groups(T, Hq, Hk);
-  return groups <= 0 || entries < 0 ? 1 : attn_waves(T, groups * Hk, entries);
+  return groups <= 0 || entries < 0 ? 1 : attn_waves(T, groups * Hk, entries, Hq / Hk);
 }
 
 extern "C" int fr_paged_attention_plan(const int32_t* kv_indices, const int32_t* kv_start,

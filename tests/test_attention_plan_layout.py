@@ -78,3 +78,10 @@ def test_split_of_prompts_over_cached_prefixes():
     assert waves([(0, 1100)]) == waves([(9000, 1100)]) > 1
     assert waves([(0, 300)] * 4) == waves([(3000, 300)] * 4) > 1
     assert waves([(129, 1)] * 2048) == load().fr_paged_attention_waves(2048, 16, 8, 2048 * 130)
+
+
+def test_rows_of_one_head_group_are_split():
+    from flashrec_amd._lib import load
+
+    w = load().fr_paged_attention_waves
+    assert w(1024, 32, 32, 1024 * 200) == 2 and w(2048, 16, 8, 2048 * 130) == 1

@@ -143,3 +143,22 @@ def test_probabilities_keep_32_bits(dev, hq, hk, waves):
     want = ((p[..., 0] - p[..., 1]) * 448)[..., None]
     err = ((got - want) / want).abs().max().item()
     assert err < 2.0 ** -8 + 2.0 ** -9, err
+
+
+@pytest.mark.parametrize("waves", [1, 2, 4])
+def test_nan_in_a_group_of_two_prompts(dev, waves):
+    """The same where the segments of a group go to the waves in turn (two and
+    more, on two waves): tokens 32 .. 44 of the first prompt share a group with
+    the second one's first; its position 40 is NaN."""
+    idx, start, lens = _case("prompts", 4)
+    g = torch.Generator().manual_seed(8)
+    k = torch.randn(4001, 8, 128, generator=g).to(E4M3)
+    v = torch.randn(4001, 8, 128, generator=g).to(E4M3)
+    q = torch.randn(lens.numel(), 16, 128, generator=g).to(torch.bfloat16)
+    clean = _run(dev, q, k, v, idx, start, lens, waves, True)
+    v.view(torch.uint8)[int(idx[40])] = 0x7F
+    got = _run(dev, q, k, v, idx, start, lens, waves, True)
+    sees = (start == start[0]) & (lens > 40)
+    assert int(sees.sum()) == 5 and bool(torch.isnan(got[sees].float()).all())
+    assert bool(torch.isfinite(got[~sees].float()).all())
+    assert (got[~sees].float() - clean[~sees].float()).abs().max().item() < 2.0 ** -7 * 5
