@@ -281,3 +281,15 @@ def test_rotary_embedding_refuses_odd_head():
     with pytest.raises((ValueError, RuntimeError)):
         rope_inplace_any(torch.zeros(2, dtype=torch.int64), torch.zeros(2, 6), torch.zeros(2, 6), 3,
                          torch.zeros(4, 3))
+
+
+def test_linear_whose_codes_are_a_parameter():
+    """A loader that registers the codes and scales as Parameters: forward_fp8 gets as far as the kernels' own check."""
+    from flashrec_amd.layers.linear import Linear
+
+    lin = Linear(32, 16)
+    lin.w_codes = torch.nn.Parameter(torch.zeros(16, 32).to(torch.float8_e4m3fn), requires_grad=False)
+    lin.w_scale = torch.nn.Parameter(torch.ones(16), requires_grad=False)
+    q = torch.zeros(4, 32).to(torch.float8_e4m3fn)
+    with pytest.raises(RuntimeError, match="ROCm"):
+        lin.forward_fp8(q, torch.ones(4, 1), (4, 32), torch.bfloat16)
