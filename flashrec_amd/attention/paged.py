@@ -301,13 +301,17 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
                               kv_indices: torch.Tensor, kv_start: torch.Tensor, kv_len: torch.Tensor,
                               scale: float, group_prefix: Optional[torch.Tensor] = None,
                               out: Optional[torch.Tensor] = None, out_scale: Optional[torch.Tensor] = None,
-                              entries: Optional[int] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+                              entries: Optional[int] = None, rows: Optional[torch.Tensor] = None
+                              ) -> Tuple[torch.Tensor, torch.Tensor]:
     """``per_token_quant_fp8(paged_attention(...).reshape(T, -1))`` in one
     kernel: the o projection's e4m3 input ``[T, Hq * D]`` and its scales
     ``[T, 1]`` (qwen3.py:131-134 -> linear.py:118-151), bit-for-bit the two
     steps' result.  Head layouts the fused kernel does not take (more than 8
     kv heads, 8 query heads per kv head), and launches with too few query
-    groups to fill the chip, run the two steps."""
+    groups to fill the chip, run the two steps; the attention's bf16 rows then go
+    to ``rows`` (contiguous, [T, Hq, D]) or, without it, to a tensor allocated
+    here, as do codes for an ``out`` with gaps between its rows.  With ``rows``,
+    ``out_scale`` and a contiguous ``out`` given nothing is allocated."""
     T, Hq, D, slots, Hk = _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len)
     if out is None:
         out = torch.empty(T, Hq * D, dtype=torch.float8_e4m3fn, device=q.device)
@@ -318,7 +322,10 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
         raise ValueError("out must be [T, Hq * D] float8_e4m3fn with a unit inner stride")
     if out_scale.dtype != torch.float32 or out_scale.numel() != T or not out_scale.is_contiguous():
         raise ValueError("out_scale must hold T contiguous fp32 values")
-    require_device(out, out_scale)
+    if rows is not None and (rows.dtype != torch.bfloat16 or tuple(rows.shape) != (T, Hq, D)
+                             or not rows.is_contiguous()):
+        raise ValueError("rows must be contiguous [T, Hq, D] bf16")
+    require_device(out, out_scale, rows)
     # where paged_attention splits its items' keys over waves, the quant runs
     # on its rows (one more launch of 3 us; 512 rows over 1503 keys take 89 us
     # fused and unsplit, 25 us so)
@@ -334,8 +341,8 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
             return out, out_scale
         except Unsupported:
             pass
-    o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, group_prefix=group_prefix,
-                        entries=entries)
+    o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, out=rows,
+                        group_prefix=group_prefix, entries=entries)
     codes = out if out.is_contiguous() else torch.empty((T, Hq * D), dtype=out.dtype, device=out.device)
     call("fr_per_token_quant_fp8", o.data_ptr(), DTYPE_CODE[o.dtype], T, Hq * D, Hq * D, codes.data_ptr(),
          out_scale.data_ptr(), stream_of(q))

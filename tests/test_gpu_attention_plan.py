@@ -150,3 +150,23 @@ def test_graph_decode_of_fewer_rows(dev, quant):
         err = (got - want).abs().amax(1) / want.abs().amax(1)
         assert err.max().item() < bound, (n, shared, err.max().item())
     be.end_graph_decode()
+
+
+@pytest.mark.parametrize("t", [40, 88])
+def test_quant_into_given_buffers_allocates_nothing(dev, t):
+    """With room for the codes, the scales and the bf16 rows, also where the keys are split (both sizes here)."""
+    from flashrec_amd._lib import load
+    from flashrec_amd.attention import attention_plan, paged_attention_quant_fp8
+
+    q, k, v, idx, start, ln = _inputs(dev, 16, 8)
+    plan = attention_plan(idx, start, ln, 16, 8)
+    assert load().fr_paged_attention_waves(t, 16, 8, idx.numel()) > 1
+    want = paged_attention_quant_fp8(q[:t], k, v, idx, start, ln, SCALE, group_prefix=plan)
+    out, scale = torch.empty_like(want[0]), torch.empty_like(want[1])
+    rows = torch.empty(t, 16, 128, dtype=torch.bfloat16, device=dev)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    paged_attention_quant_fp8(q[:t], k, v, idx, start, ln, SCALE, group_prefix=plan, out=out, out_scale=scale, rows=rows)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+    assert torch.equal(out.view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(scale, want[1])
+    with pytest.raises(ValueError, match="rows"):
+        paged_attention_quant_fp8(q[:t], k, v, idx, start, ln, SCALE, out=out, out_scale=scale, rows=rows[1:])
