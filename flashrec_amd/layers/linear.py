@@ -110,17 +110,11 @@ class Linear(nn.Module):
     def _fp8_scale(self) -> Optional[torch.Tensor]:
         return self.w_scale
 
-    def _held(self, name: str) -> Optional[torch.Tensor]:
-        """The attribute ``name``, from the module's dict of buffers where it is
-        one (Module.__getattr__ costs most of a microsecond); a loader may have
-        put a Parameter in its place."""
-        buffers = self._buffers
-        return buffers[name] if name in buffers else getattr(self, name)
-
     def _prearranged(self) -> PrearrangedFp8Weight:
         """The codes in the prearranged GEMM's layout, built when first needed
         on the codes' device (and kept until the weights change or move)."""
-        cached, codes = self.__dict__.get("_pre"), self._held("w_codes")
+        buffers = self._buffers
+        cached, codes = self.__dict__.get("_pre"), buffers["w_codes"] if "w_codes" in buffers else self.w_codes
         if cached is None or cached.data.get_device() != codes.get_device():
             cached = prearrange_fp8_weight(codes.t())
             self.__dict__["_pre"] = cached
@@ -212,7 +206,11 @@ class Linear(nn.Module):
         """GEMM of already quantised ``[M, K]`` e4m3 rows with their ``[M, 1]``
         scales; the result has shape ``orig_shape[:-1] + (out_features,)``
         (linear.py:134-142, 153-172)."""
-        codes, scale, bias = self._held("w_codes"), self._held("w_scale"), self.bias
+        # from the module's dict where they are buffers (Module.__getattr__ costs
+        # most of a microsecond); a loader may have put Parameters in their place
+        buffers, bias = self._buffers, self.bias
+        codes = buffers["w_codes"] if "w_codes" in buffers else self.w_codes
+        scale = buffers["w_scale"] if "w_scale" in buffers else self.w_scale
         if codes is None:
             raise RuntimeError("Linear.forward_fp8 needs fp8 weights (load an fp8 checkpoint "
                                "or pass quantize_fp8=True)")
