@@ -243,18 +243,15 @@ def attention_plan(kv_indices: torch.Tensor, kv_start: torch.Tensor, kv_len: tor
     require_device(kv_indices, kv_start, kv_len)
     T = int(kv_start.numel())
     groups, stride = _groups(T, hq, hk)
-    plan = out
-    if out is None or not _plan_records(out, groups, stride):
-        if out is not None:
-            _check_plan_buffer(out, groups, False)
-        plan = torch.empty(max(groups, 1) * stride, dtype=torch.int32, device=kv_start.device)
+    if out is None:
+        plan = rows = torch.empty((max(groups, 1), stride), dtype=torch.int32, device=kv_start.device).select(1, 0)
     else:
-        _check_plan_buffer(out, groups, True)
+        records = _plan_records(out, groups, stride)
+        _check_plan_buffer(out, groups, records)
+        plan = out if records else torch.empty(groups * stride, dtype=torch.int32, device=kv_start.device)
+        rows = out if out.dim() == 1 and out.stride(0) == stride else _plan_rows(plan, T, hq, hk)
     call("fr_paged_attention_plan", kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
          T, int(hq), int(hk), plan.data_ptr(), stream_of(kv_start))
-    if plan is out and out.stride(-1) == stride:
-        return out
-    rows = _plan_rows(plan, T, hq, hk)
     if out is not None and plan is not out:
         out.view(-1)[:groups].copy_(rows)
         return out
@@ -329,7 +326,9 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     # where paged_attention splits its items' keys over waves, the quant runs
     # on its rows (one more launch of 3 us; 512 rows over 1503 keys take 89 us
     # fused and unsplit, 25 us so)
-    if _waves(T, Hq, Hk, kv_indices, entries) == 1:
+    waves = _waves(T, Hq, Hk, kv_indices, entries)
+    plan = _check_plan(group_prefix, T, Hq, Hk)
+    if waves == 1:
         try:
             call("fr_paged_attention_quant_fp8",
                  q.data_ptr(), q.stride(0), q.stride(1),
@@ -337,12 +336,12 @@ def paged_attention_quant_fp8(q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
                  v_cache.data_ptr(), v_cache.stride(0), v_cache.stride(1),
                  slots, kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
                  out.data_ptr(), out.stride(0), out_scale.data_ptr(),
-                 T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk), stream_of(q))
+                 T, Hq, Hk, D, float(scale), plan, stream_of(q))
             return out, out_scale
         except Unsupported:
             pass
-    o = paged_attention(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, out=rows,
-                        group_prefix=group_prefix, entries=entries)
+    o = torch.empty(T, Hq, D, dtype=torch.bfloat16, device=q.device) if rows is None else rows
+    _attend(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, o, plan, waves)
     codes = out if out.is_contiguous() else torch.empty((T, Hq * D), dtype=out.dtype, device=out.device)
     call("fr_per_token_quant_fp8", o.data_ptr(), DTYPE_CODE[o.dtype], T, Hq * D, Hq * D, codes.data_ptr(),
          out_scale.data_ptr(), stream_of(q))
@@ -369,12 +368,19 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     T, Hq, D, slots, Hk = _check_attention_inputs(q, k_cache, v_cache, kv_indices, kv_start, kv_len)
     if out is None:
         out = torch.empty(T, Hq, D, dtype=torch.bfloat16, device=q.device)
+    _attend(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, out, _check_plan(group_prefix, T, Hq, Hk),
+            _waves(T, Hq, Hk, kv_indices, entries))
+    return out
+
+
+def _attend(q, k_cache, v_cache, kv_indices, kv_start, kv_len, scale, out, plan: int, waves: int) -> None:
+    """The launch, with inputs and plan checked."""
+    T, Hq, D = q.shape
+    slots, Hk, _ = k_cache.shape
     call("fr_paged_attention_split_fp8",
          q.data_ptr(), q.stride(0), q.stride(1),
          k_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
          v_cache.data_ptr(), v_cache.stride(0), v_cache.stride(1),
          slots, kv_indices.data_ptr(), kv_start.data_ptr(), kv_len.data_ptr(),
          out.data_ptr(), out.stride(0), out.stride(1),
-         T, Hq, Hk, D, float(scale), _check_plan(group_prefix, T, Hq, Hk),
-         _waves(T, Hq, Hk, kv_indices, entries), stream_of(q))
-    return out
+         T, Hq, Hk, D, float(scale), plan, waves, stream_of(q))
