@@ -953,8 +953,8 @@ extern "C" int fr_paged_attention_quant_fp8(const void* q, int64_t sqt, int64_t 
   const int rc = attn_args(a, q, sqt, sqh, k_cache, skp, skh, v_cache, svp, svh, num_slots, kv_indices, kv_start,
                            kv_len, T, Hq, Hk, D, scale, group_prefix);
   if (rc != FR_OK) return rc;
-  // one wave per kv head in a workgroup of 8; 8-wide query groups take the
-  // token path in a kernel of their own, which this fusion does not cover
+  // one wave per kv head in a workgroup of 8; the quantizing passes hold a token
+  // of up to 32 heads, which 8 query heads for each of 8 kv heads would pass
   if (Hk > 8 || Hq / Hk == 8) return FR_EUNSUPPORTED;
   if (T == 0) return FR_OK;
   if (!out_q || !out_scale || ldq < Hq * D) return FR_EINVAL;

@@ -35,7 +35,8 @@
 //     and the advanced trie nodes.
 // 8 x 512 beams x 1024 candidates -> top 512: 34.0 + 33.6 us with merge trees,
 // 18.2 + 18.3 so; 1 x 512 33.6 + 33.7 -> 15.4 + 17.8; 8 x 35 21.4 + 10.6 -> 10.1
-// + 8.4.  What is left is latency: kernel 2 is one CU per request.
+// + 8.4, both together 5.6 less with narrow beams and few lists told apart (below).
+// What is left is latency: kernel 2 is one CU per request.
 #include <mutex>
 #include <type_traits>
 
