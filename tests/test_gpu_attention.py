@@ -39,7 +39,7 @@ def _run(dev, q, k, v, idx, start, ln):
 
 @pytest.mark.parametrize("hq,hk", [(16, 8), (8, 8), (16, 4), (16, 2)])
 def test_decode_ragged(dev, hq, hk):
-    """Rows of 1 .. 1000 keys (across and inside the 8 * NP key chunks)."""
+    """Rows of 1 .. 1000 keys (across and inside the 32-key blocks)."""
     lens = [1, 2, 7, 8, 9, 63, 64, 65, 128, 130, 257, 1000]
     slots = 4096
     k, v = _pool(slots, hk, hq + hk)

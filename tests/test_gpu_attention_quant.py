@@ -4,9 +4,9 @@
 Bar: bit-exact against the two steps it replaces, the attention kernel
 (itself held to the oracle in test_gpu_attention.py) followed by
 ``per_token_quant_fp8`` on its bf16 output, codes and scales alike, on the
-shared-prefix (MFMA) groups, the token-by-token groups, partial last groups,
-empty rows, strided queries and output rows, with and without the plan, and
-at config 4's full size.  Head layouts the fused kernel refuses take the two
+shared-prefix groups, groups of several segments, partial last groups, empty
+rows, strided queries and output rows, with and without the plan, and at config
+4's full size.  Head layouts the fused kernel refuses take the two
 steps and must give the same bits too."""
 
 import pytest
@@ -83,7 +83,7 @@ def test_shared_prefix_beams(dev, hq, hk, plan):
 
 @pytest.mark.parametrize("hq,hk", [(16, 8), (16, 2), (8, 8)])
 def test_token_path_ragged(dev, hq, hk):
-    """No shared prefix: every group goes token by token; 1 .. 1000 keys."""
+    """No shared prefix: every token a segment of its own; 1 .. 1000 keys."""
     lens = [1, 2, 7, 8, 9, 63, 64, 65, 128, 130, 257, 1000, 5, 17, 33, 40, 31, 3]
     slots = 4096
     k, v = _pool(slots, hk, 40 + hq)
@@ -167,3 +167,36 @@ def test_config4_full_size(dev):
                        for r in rows.tolist()])
     err = ((att.cpu()[rows].float() - ref.float()).abs().amax(-1) / ref.float().abs().amax(-1).clamp(min=1e-6))
     assert err.max().item() < 1e-2
+
+
+@pytest.mark.parametrize("hq,hk", [(16, 8), (8, 8), (16, 4), (4, 1)])
+@pytest.mark.parametrize("kind", ["prompts", "beams", "rows"])
+def test_fused_kernel_on_segments(dev, kind, hq, hk):
+    """The fused kernel itself (the wrapper takes it for launches that fill the
+    chip only) on groups of several segments, empty rows and a partial last
+    group, with and without the plan: bit-exact with the unsplit attention
+    kernel followed by the quant; bytes past each row stay as they were."""
+    from flashrec_amd._lib import call
+    from flashrec_amd.attention import attention_plan
+    from flashrec_amd.kernel.sglops import per_token_quant_fp8
+    from test_gpu_attention_split import _case, _run
+
+    print(f"fused {kind} {hq}/{hk}", flush=True)
+    idx, start, ln = _case(kind, 3)
+    t = int(ln.numel())
+    k, v = _pool(4001, hk, 90 + hq)
+    q = torch.randn(t, hq, 128, generator=torch.Generator().manual_seed(91)).to(torch.bfloat16)
+    d = [x.to(dev) for x in (q, k, v, idx, start, ln)]
+    plan = attention_plan(d[3], d[4], d[5], hq, hk)
+    for gp in (None, plan):
+        ref_q, ref_s = per_token_quant_fp8(_run(dev, q, k, v, idx, start, ln, 1, gp is not None).to(dev).reshape(t, -1))
+        codes = torch.full((t + 1, hq * 128 + 64), 0x55, dtype=torch.uint8, device=dev)
+        scales = torch.full((t + 1,), 7.0, device=dev)
+        call("fr_paged_attention_quant_fp8", d[0].data_ptr(), hq * 128, 128, d[1].data_ptr(), hk * 128, 128,
+             d[2].data_ptr(), hk * 128, 128, 4001, d[3].data_ptr(), d[4].data_ptr(), d[5].data_ptr(),
+             codes.data_ptr(), hq * 128 + 64, scales.data_ptr(), t, hq, hk, 128, SCALE,
+             0 if gp is None else gp.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(codes[:t, : hq * 128].cpu(), ref_q.view(torch.uint8).cpu())
+        assert torch.equal(scales[:t].view(torch.int32).cpu(), ref_s.view(-1).view(torch.int32).cpu())
+        assert bool((codes[:, hq * 128:] == 0x55).all()) and bool((codes[t] == 0x55).all()) and float(scales[t]) == 7.0
