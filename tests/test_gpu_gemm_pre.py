@@ -34,7 +34,8 @@ def _same_values(a, b):
 
 
 # config shapes (gate_up at 4096 and 512 rows, down, qkv, o, the SID head) and
-# edge shapes: partial tiles, N not a multiple of 32, K tails of every kind
+# edge shapes, of few tiles (the K-split kernel): partial tiles, N not a multiple
+# of 32, K tails of every kind; the large tiles' edges are at the end
 SHAPES = [(4096, 12288, 2048), (512, 12288, 2048), (4096, 2048, 6144), (4096, 4096, 2048), (4096, 2048, 2048),
           (300, 1000, 384), (33, 200, 320), (1, 256, 2048), (257, 264, 48), (64, 512, 1024)]
 
@@ -138,3 +139,14 @@ def test_prearranged_rejects_mismatched_k(dev):
     with pytest.raises(ValueError):
         fp8_scaled_mm_prearranged(torch.zeros(4, 128, dtype=torch.float8_e4m3fn, device=dev), w,
                                   torch.ones(4, 1, device=dev), torch.ones(64, device=dev))
+
+
+# ragged rows and columns and K tails on the large tiles (shapes of fewer tiles
+# take the K-split kernel): 256x256 in two rounds and one, 256x128 in two and one,
+# 128x128 in two and one; the first 192x128 in the plain layout
+@pytest.mark.parametrize("m,n,k", [(1300, 12272, 272), (4100, 2032, 272), (2661, 6128, 336), (520, 12272, 336),
+                                   (3685, 2160, 656), (1000, 2032, 1040)])
+def test_large_tile_edges_exact(dev, m, n, k):
+    from test_gpu_gemm_small import test_small_gemm_exact
+
+    test_small_gemm_exact(dev, m, n, k)

@@ -6,11 +6,11 @@ the fp32 dequantised oracle in test_gpu_gemm.py) rounded to the residual's
 dtype, then the residual add in that dtype (torch's bf16 / fp16 add, which
 rounds the fp32 sum once: the reference's ``residual + x``,
 sglops.py:53-55).  Covered: the decode step's o and down shapes (the
-256 x 128 tile's fast epilogue), edge tiles and tails (the bounds-checked
-path), the 256 x 256 tile (which routes the add through the bounds-checked
-path), the 192 x 128 and 128 x 128 tiles and several tiles per workgroup
-(M = 512, 1381 and 2661 rows), fp16, in place and into a separate buffer, a
-strided residual."""
+256 x 128 tile's fast epilogue), launches of few tiles (the K-split kernel),
+the 256 x 256 tile (which routes the add through the bounds-checked path), the
+192 x 128 tile and several tiles per workgroup (M = 512, 1381 and 2661 rows),
+fp16, in place and into a separate buffer, a strided residual.  (The large
+tiles' edges, the 128 x 128 tile's among them: test_gpu_gemm_pre.py.)"""
 
 import pytest
 import torch

@@ -14,7 +14,7 @@ Bars:
   silu_and_mul_per_token_quant_fp8 of the GPU's gate_up output, at the fp8
   parity bar.
 Shapes: the decode step's gate_up (256 x 256 tile), M = 512 (256 x 128),
-small N (128 x 128), ragged M and N (the bounds-checked path), M = 1, K not
+few tiles (the K-split kernel), ragged M and N, M = 1, K not
 a multiple of 16 (operands repacked by the wrapper), and several tiles per
 workgroup on the 256 x 128 and 128 x 128 tiles."""
 
